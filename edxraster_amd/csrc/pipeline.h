@@ -274,7 +274,7 @@ struct DeviceBuffers {
 // mesh; light is w.r.t. the light direction as given, material is (ambient,
 // kd, ks, shininess).
 // The per-vertex sums are accumulated in double first: jobs that share their
-// vertex outputs share one accumulator of 9 x acc_v doubles (value-major) at
+// vertex outputs share one accumulator of 9 x acc_v doubles (vertex-major) at
 // acc_base, which the first of them (group_first) adds to the outputs at the
 // end.
 struct GradPtrs {
@@ -303,10 +303,11 @@ hipError_t set_frame_job(hipGraphExec_t exec, hipGraphNode_t first, const BatchP
 // Adjoint of the shading of a rendered batch with visibility held fixed (the
 // triangle-ID buffer): d_rgb holds dLoss/d(clamped float RGB) per pixel in the
 // layout of color_f32; acc is 8 doubles of scratch per job, vacc the vertex
-// accumulators (vacc_size doubles, the GradPtrs' acc_base ranges).
+// accumulators (vacc_size doubles, vertex-major in the GradPtrs' acc_base
+// ranges); any_pow: a job's shininess is no whole exponent.
 hipError_t launch_adjoint(const BatchParams& Q, const FrameParams* jobs, const GradPtrs* grads,
                           const uint32_t* ids, const float* d_rgb, double* acc,
-                          double* vacc, uint64_t vacc_size, hipStream_t s);
+                          double* vacc, uint64_t vacc_size, bool any_pow, hipStream_t s);
 // Kernel attributes (dynamic LDS limits) and occupancy; once per process before launches.
 hipError_t init_kernels();
 
