@@ -187,7 +187,7 @@ struct edxr_ctx {
     DevBuf<RasterRec> rrec;
     DevBuf<ShadeRec> srec;
     DevBuf<uint32_t> desc, clipQueue, binCounts, tileTotals, tileStart, refs, counters, color, ids, work, tileItem,
-        tileBig;
+        tileBig, tileSums;
     DevBuf<float> depth;
     DevBuf<uint64_t> partials;
     DevBuf<uint32_t> chunkBox;
@@ -477,7 +477,8 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
     if ((e = c->jobsDev.ensure(Q.num_jobs)) != hipSuccess ||
         (e = c->tileTotals.ensure(Q.total_tiles)) != hipSuccess ||
         (e = c->tileStart.ensure((size_t)Q.total_tiles + 1)) != hipSuccess ||
-        (e = c->tileItem.ensure(Q.total_tiles)) != hipSuccess || (e = c->tileBig.ensure(Q.total_tiles)) != hipSuccess)
+        (e = c->tileItem.ensure(Q.total_tiles)) != hipSuccess || (e = c->tileBig.ensure(Q.total_tiles)) != hipSuccess ||
+        (e = c->tileSums.ensure((size_t)(Q.total_tiles / kTileBlock + 1) * kTileSumWords)) != hipSuccess)
         return c->hip_fail(e, "hipMalloc(job tables)");
     if (!single) {
         if ((e = c->jobsHost.ensure(Q.num_jobs)) != hipSuccess) return c->hip_fail(e, "hipHostMalloc(jobs)");
@@ -560,6 +561,7 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
         B.work_cap = (uint32_t)c->work.cap;
         B.tile_item = c->tileItem.p;
         B.tile_big = c->tileBig.p;
+        B.tile_sums = c->tileSums.p;
         B.partials = c->partials.p;
         B.raster_blocks = rasterBlocks;
         // The persistent raster grid is the resident capacity: workgroups
@@ -818,7 +820,7 @@ void edxr_destroy(edxr_ctx* c) {
     c->rrec.release();
     c->srec.release();
     for (DevBuf<uint32_t>* b : {&c->desc, &c->clipQueue, &c->binCounts, &c->tileTotals, &c->tileStart, &c->refs,
-                                &c->counters, &c->color, &c->ids, &c->work, &c->tileItem, &c->tileBig, &c->groupSums,
+                                &c->counters, &c->color, &c->ids, &c->work, &c->tileItem, &c->tileBig, &c->tileSums, &c->groupSums,
                                 &c->jobTables, &c->bcolor, &c->bids})
         b->release();
     c->depth.release();
@@ -1062,6 +1064,9 @@ int edxr_render_mesh_noalloc(edxr_ctx* c, const edxr_mesh* m, void* color, void*
         B.scan_spin_limit = kScanSpinLimit;
         B.legacy_scans = legacyScans ? 1u : 0u;
         B.clip_queue = s.take<uint32_t>(clipCap);
+        // The tile scan comes after the clip stage: its sums take the queue's place.
+        static_assert((kMaxTiles / kTileBlock) * kTileSumWords <= 1024, "the clip queue holds 1024 entries at least");
+        B.tile_sums = B.clip_queue;
         B.bin_counts = s.take<uint32_t>(countEntries);
         B.refs = s.take<uint32_t>(refCap);
         B.work = s.take<uint32_t>(workCap);

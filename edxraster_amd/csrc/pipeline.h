@@ -21,7 +21,7 @@ constexpr int kMaxPoly = 16;                 // clip polygon capacity (convex in
 constexpr uint32_t kMaxSampleLevel = 5;      // up to 32 samples per pixel
 constexpr uint32_t kPassSamples = 4;         // samples whose keys one raster pass keeps in LDS
 constexpr uint32_t kSegLog2Min = 8;          // raster work items hold 256 .. 4096 tile references,
-constexpr uint32_t kSegLog2Max = 12;         // chosen per frame from the total (k_bin_tilescan)
+constexpr uint32_t kSegLog2Max = 12;         // chosen per frame from the total (frame_seg_log2)
 constexpr uint32_t kSegRefs = 1u << kSegLog2Max;
 // Tiles whose references are mostly tile-level triangles (each takes a whole
 // wave in the raster) are cut into segments of 2^kSegLog2Heavy references when
@@ -33,8 +33,12 @@ constexpr uint32_t kHeavyBigMin = 32;
 constexpr uint32_t kImageBits = 26;
 constexpr uint32_t kImageMask = (1u << kImageBits) - 1;
 constexpr uint32_t kChunkGroup = 64;         // chunks per block of the column scan
-constexpr uint32_t kTilescanStaged = 8192;   // batch tiles whose counts k_bin_tilescan stages in LDS
-constexpr uint32_t kTilescanWork = 8192;     // work items k_bin_tilescan stages in LDS (with the tiles)
+// Tiles that the one-workgroup tile scan takes: it needs 9.5 us for 3,600 (17
+// us for 8,160 before it was confined to these), the two launches that take
+// more tiles 10 to 12 us at any size.
+constexpr uint32_t kTilescanOne = 4096;
+constexpr uint32_t kTileBlock = 1024;        // tiles per workgroup of the two launches
+constexpr uint32_t kTileSumWords = 16;       // words of a workgroup's sums between them
 constexpr uint32_t kScanSpinLimit = 1u << 20;  // k_bin_colpass look-back waits (about 30 ms) before giving up
 // Single-sample shading rebuilds a winner's screen values from its shading
 // vertices, instead of gathering them, in tiles of this many references or
@@ -209,7 +213,9 @@ enum CounterSlot {
     kCntSegLog2,         // log2 of the tile references per work item of this frame
     kCntStriped = 16,    // high-rate counters: kStripes slots each, summed on the host
     kCntAllocStriped = kCntStriped + 4 * 32,  // k_clip's allocations: kAllocStripes vertices, then records
-    kCntSlots = kCntAllocStriped + 2 * 16
+    kCntTileRefs = kCntAllocStriped + 2 * 16,  // tile references and deepest tile, kAllocStripes each
+    kCntTileDeepest = kCntTileRefs + 16,       // (frames of more than kTilescanOne tiles)
+    kCntSlots = kCntTileDeepest + 16
 };
 
 // Counters bumped by many workgroups are striped over kStripes addresses so
@@ -256,6 +262,7 @@ struct DeviceBuffers {
     uint32_t* work;        // raster work items: global tile | segment << kTileBits | kSingleSegment
     uint32_t work_cap;
     uint32_t* tile_item;   // per global tile: first key image (one per segment) | segment log2 << kImageBits
+    uint32_t* tile_sums;   // kTileSumWords per kTileBlock tiles (frames of more than kTilescanOne tiles)
     uint32_t* tile_big;    // per global tile: heavy references (big, or compact with kDescHeavy)
     uint64_t* partials;    // work_cap * samples * 1024 (depth, order) keys, one tile image per item and sample
     uint32_t raster_blocks;  // work items the segment size is chosen for

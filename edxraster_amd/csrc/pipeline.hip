@@ -16,7 +16,7 @@
 //                (Core/Clipper.h:109-170,192-288).
 //   k_bin_count  per-chunk tile histograms (binning, Core/Renderer.cpp:161-230)
 //   k_bin_colpass (or k_bin_colsum / k_bin_groupscan / k_bin_colscan) and
-//   k_bin_tilescan
+//   k_bin_tilescan (or k_bin_tilesums / k_bin_tileplace)
 //                exclusive scans -> per-(tile, chunk) offsets and the raster
 //                work list of (tile, segment) items.
 //   k_bin_scatter scatter through LDS cursors: a tile's list holds the chunks'
@@ -1054,6 +1054,17 @@ __device__ __forceinline__ void colgroup_range(const FrameParams& P, uint32_t& c
 }
 }  // namespace
 
+namespace {
+// A wave's tiles' references and deepest tile, added to the frame's striped counters.
+__device__ __forceinline__ void tile_stats_add(const DeviceBuffers& B, uint32_t n, uint32_t stripe) {
+    const uint32_t sum = wave_sum(n), deep = wave_max(n);
+    if (__lane_id() == 0 && sum) {
+        atomicAdd(&B.counters[kCntTileRefs + stripe % kAllocStripes], sum);
+        atomicMax(&B.counters[kCntTileDeepest + stripe % kAllocStripes], deep);
+    }
+}
+}  // namespace
+
 // Whether block (x, y) of the column-scan grid lies inside job P's matrix.
 __device__ __forceinline__ bool colgroup_in_job(const FrameParams& P) {
     return blockIdx.x * kWave < P.num_tiles && blockIdx.y * kChunkGroup < P.num_chunks;
@@ -1079,8 +1090,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_groupscan(BatchParams Q, const F
                                                           DeviceBuffers B) {
     const FrameParams& P = jobs[blockIdx.z];
     const uint32_t tile = blockIdx.x * kBlock + threadIdx.x;
-    if (tile >= P.num_tiles) return;
-    const uint32_t G = (P.num_chunks + kChunkGroup - 1) / kChunkGroup;
+    const bool in = tile < P.num_tiles;
+    const uint32_t G = in ? (P.num_chunks + kChunkGroup - 1) / kChunkGroup : 0u;
     uint32_t* col = &B.group_sums[P.group_base + tile];
     uint32_t run = 0;
     // Batches of 16 groups: the loads of a batch are issued before its stores.
@@ -1095,7 +1106,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_groupscan(BatchParams Q, const F
             run += v[k];
         }
     }
-    B.tile_totals[P.tile_base + tile] = run;
+    if (in) B.tile_totals[P.tile_base + tile] = run;
+    if (Q.total_tiles > kTilescanOne) tile_stats_add(B, run, blockIdx.x);
 }
 
 // Step 3: rewrite the counts in place as offsets within the tile's list.
@@ -1202,6 +1214,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_colpass(BatchParams Q, const Fra
             status_store(st + (size_t)g * P.num_tiles, kInclusive | ((excl + groupTotal) & kStatusValue));
             if (g == G - 1) B.tile_totals[P.tile_base + tile] = excl + groupTotal;
         }
+        if (g == G - 1 && Q.total_tiles > kTilescanOne) tile_stats_add(B, in ? excl + groupTotal : 0u, x);
         sExcl[lane] = excl;
     }
     __syncthreads();
@@ -1247,45 +1260,103 @@ __device__ __forceinline__ uint32_t tile_segments(uint32_t n, uint32_t segLog2) 
 }
 }  // namespace
 
-// Exclusive scan of the tile totals over every job's tiles (global tiles <=
-// 2^18, one block of 1024), and the raster work list: one item per (tile,
-// segment of <= 2^segLog2 refs).  The segment size is the smallest of 256 ..
-// 4096 that gives no more items than the raster grid has workgroups (beyond
-// one per tile), so a frame with few references is still spread over the
-// whole grid instead of being bound by one workgroup walking a deep tile.
-// Items are listed longest first, so that the last ones claimed are short and
-// the pass does not end on one workgroup finishing a full segment: every full
-// segment, then the tiles' last (partial) segments in four size classes,
-// largest first.  A segment's key image is at the tile's image base
-// (tile_item) plus its segment index, whatever its place in the list.
+namespace {
+// log2 of the frame's references per work item, and whether every tile's
+// segment indices then fit a work item.
+__device__ __forceinline__ uint32_t frame_seg_log2(uint32_t total, uint32_t deepest, uint32_t rasterBlocks, bool& fit) {
+    uint32_t segLog2 = kSegLog2Min;
+    while (segLog2 < kSegLog2Max && (total >> segLog2) > rasterBlocks) segLog2++;
+    // a tile's segment index must fit above the tile bits of a work item
+    while (segLog2 < kSegLog2Max && tile_segments(deepest, segLog2) > (1u << kSegIndexBits)) segLog2++;
+    fit = tile_segments(deepest, segLog2) <= (1u << kSegIndexBits);
+    return segLog2;
+}
+
+// A tile's segment log2: the frame's, or kSegLog2Heavy for a tile whose
+// references are mostly tile-level triangles (a whole wave each), so that
+// such a tile is spread over several workgroups.  Finer segments never
+// make a tile's segment index overflow its bits.
+__device__ __forceinline__ uint32_t tile_seg_log2(uint32_t n, uint32_t big, uint32_t segLog2, bool split) {
+    if (!split || big < kHeavyBigMin || 4 * big < n) return segLog2;
+    uint32_t s = kSegLog2Heavy;
+    while (s < segLog2 && tile_segments(n, s) > (1u << kSegIndexBits)) s++;
+    return s;
+}
+
+// Adds a tile's full segments (cnt[0]) and its partial last segment by size
+// class (cnt[1 + c], class c = remainder >> (the tile's segment log2 - 2)).
+__device__ __forceinline__ void count_segments(uint32_t n, uint32_t s, uint32_t (&cnt)[5]) {
+    cnt[0] += n >> s;
+    const uint32_t r = n & ((1u << s) - 1);
+    if (r) {
+        // (an array index known at compile time keeps cnt in registers)
+        const uint32_t c = r >> (s - 2);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) cnt[1 + k] += c == k ? 1u : 0u;
+    }
+}
+
+// The first list position of each class: full segments, then classes 3, 2, 1, 0.
+__device__ __forceinline__ void class_starts(const uint32_t (&tot)[5], uint32_t (&pos)[5]) {
+    pos[0] = 0;
+    pos[4] = tot[0];
+    pos[3] = pos[4] + tot[4];
+    pos[2] = pos[3] + tot[3];
+    pos[1] = pos[2] + tot[2];
+}
+
+// A tile's work items, at its classes' next positions; returns its segments.
+__device__ __forceinline__ uint32_t place_tile(uint32_t* work, uint32_t t, uint32_t n, uint32_t s, uint32_t (&pos)[5]) {
+    const uint32_t nf = n >> s, r = n & ((1u << s) - 1);
+    const uint32_t segs = nf + (r ? 1u : 0u);
+    // a tile of one segment is marked (kSingleSegment): its image is the
+    // 32-bit winner orders
+    const uint32_t single = segs == 1 ? kSingleSegment : 0u;
+    for (uint32_t i = 0; i < nf; i++) work[pos[0]++] = t | (i << kTileBits) | single;
+    if (r) {
+        const uint32_t c = r >> (s - 2);
+        work[c == 0 ? pos[1] : c == 1 ? pos[2] : c == 2 ? pos[3] : pos[4]] = t | (nf << kTileBits) | single;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) pos[1 + k] += c == k ? 1u : 0u;
+    }
+    return segs;
+}
+}  // namespace
+
+// Exclusive scan of the tile totals over every job's tiles and the raster work
+// list: one item per (tile, segment of <= 2^segLog2 refs).  The segment size
+// is the smallest of 256 .. 4096 that gives no more items than the raster grid
+// has workgroups (beyond one per tile), so a frame with few references is
+// still spread over the whole grid instead of being bound by one workgroup
+// walking a deep tile.  Items are listed longest first, so that the last ones
+// claimed are short and the pass does not end on one workgroup finishing a
+// full segment: every full segment, then the tiles' last (partial) segments in
+// four size classes, largest first.  A segment's key image is at the tile's
+// image base (tile_item) plus its segment index, whatever its place in the
+// list.
+// One workgroup for frames of up to kTilescanOne tiles (k_bin_tilescan), kPer
+// = 1, 2 or 4 tiles per thread in registers (475 tiles 5 us; 2,040 tiles at 2
+// per thread 6.7, at 4 8.4 us); beyond, a workgroup per kTileBlock tiles in two launches
+// (k_bin_tilesums, k_bin_tileplace), with the same outputs.
+template <uint32_t kPer>
 __global__ __launch_bounds__(1024) void k_bin_tilescan(BatchParams Q, DeviceBuffers B) {
-    // staged: [nt] totals, then [nt] big counts (overwritten by each tile's
-    // start and item entry), then up to kTilescanWork work items
-    extern __shared__ uint32_t sTiles[];
     __shared__ uint32_t sScan6[6][16];
     __shared__ uint32_t sMax, sTotal, sSegs, sExtra;
     const uint32_t nt = Q.total_tiles;
-    const uint32_t per = (nt + 1023) / 1024;
-    const uint32_t t0 = min(nt, threadIdx.x * per), t1 = min(nt, t0 + per);
     if (threadIdx.x == 0) sMax = sTotal = sSegs = sExtra = 0;
-    // Up to kTilescanStaged tiles, the totals and big counts are staged in LDS
-    // with coalesced loads that are all in flight together; the passes below
-    // walk each thread's contiguous tiles several times.
-    const bool staged = nt <= kTilescanStaged;
-    if (staged) {
-        for (uint32_t t = threadIdx.x; t < nt; t += 1024) {
-            sTiles[t] = B.tile_totals[t];
-            sTiles[nt + t] = B.tile_big[t];
-        }
+    uint32_t n[kPer], big[kPer];
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; u++) {
+        const uint32_t t = threadIdx.x * kPer + u;
+        n[u] = t < nt ? B.tile_totals[t] : 0u;
+        big[u] = t < nt ? B.tile_big[t] : 0u;
     }
     __syncthreads();
-    auto total_of = [&](uint32_t t) { return staged ? sTiles[t] : B.tile_totals[t]; };
-    auto big_of = [&](uint32_t t) { return staged ? sTiles[nt + t] : B.tile_big[t]; };
     uint32_t localRefs = 0, localMax = 0;
-    for (uint32_t t = t0; t < t1; t++) {
-        const uint32_t n = total_of(t);
-        localRefs += n;
-        localMax = max(localMax, n);
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; u++) {
+        localRefs += n[u];
+        localMax = max(localMax, n[u]);
     }
     // Total and deepest tile: wave reductions, then one LDS atomic per wave.
     const uint32_t waveRefs = wave_sum(localRefs), waveMax = wave_max(localMax);
@@ -1294,102 +1365,52 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(BatchParams Q, DeviceBuff
         atomicMax(&sMax, waveMax);
     }
     __syncthreads();
-    const uint32_t total = sTotal, maxN = sMax;
-    uint32_t segLog2 = kSegLog2Min;
-    while (segLog2 < kSegLog2Max && (total >> segLog2) > B.raster_blocks) segLog2++;
-    // a tile's segment index must fit above the tile bits of a work item
-    while (segLog2 < kSegLog2Max && tile_segments(maxN, segLog2) > (1u << kSegIndexBits)) segLog2++;
-    const bool segsFit = tile_segments(maxN, segLog2) <= (1u << kSegIndexBits);
-    // A tile's segment log2: the frame's, or kSegLog2Heavy for a tile whose
-    // references are mostly tile-level triangles (a whole wave each), so that
-    // such a tile is spread over several workgroups.  Finer segments never
-    // make a tile's segment index overflow its bits.
-    auto tile_log2 = [&](uint32_t n, uint32_t big, bool split) {
-        if (!split || big < kHeavyBigMin || 4 * big < n) return segLog2;
-        uint32_t s = kSegLog2Heavy;
-        while (s < segLog2 && tile_segments(n, s) > (1u << kSegIndexBits)) s++;
-        return s;
-    };
+    const uint32_t total = sTotal;
+    bool segsFit;
+    const uint32_t segLog2 = frame_seg_log2(total, sMax, B.raster_blocks, segsFit);
     // The finer segments of heavy tiles are taken only while the work list
     // has room for them: segments with and without them, summed over the block.
-    {
-        uint32_t segs = 0, extra = 0;
-        auto add = [&](uint32_t n, uint32_t big) {
-            const uint32_t plain = tile_segments(n, segLog2);
-            segs += plain;
-            extra += tile_segments(n, tile_log2(n, big, true)) - plain;
-        };
-        for (uint32_t t = t0; t < t1; t++) add(total_of(t), big_of(t));
-        segs = wave_sum(segs);
-        extra = wave_sum(extra);
-        if (__lane_id() == 0) {
-            atomicAdd(&sSegs, segs);
-            atomicAdd(&sExtra, extra);
-        }
-        __syncthreads();
+    uint32_t segs = 0, extra = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; u++) {
+        const uint32_t plain = tile_segments(n[u], segLog2);
+        segs += plain;
+        extra += tile_segments(n[u], tile_seg_log2(n[u], big[u], segLog2, true)) - plain;
     }
+    segs = wave_sum(segs);
+    extra = wave_sum(extra);
+    if (__lane_id() == 0) {
+        atomicAdd(&sSegs, segs);
+        atomicAdd(&sExtra, extra);
+    }
+    __syncthreads();
     const bool split = (uint64_t)sSegs + sExtra <= B.work_cap;
-    // Per thread: full segments (cnt[0]) and partial last segments by size
-    // class (cnt[1 + c], class c = remainder >> (the tile's segment log2 - 2)).
-    uint32_t cnt[5] = {0, 0, 0, 0, 0};
-    auto count = [&](uint32_t n, uint32_t big) {
-        const uint32_t s = tile_log2(n, big, split);
-        cnt[0] += n >> s;
-        const uint32_t r = n & ((1u << s) - 1);
-        if (r) cnt[1 + (r >> (s - 2))]++;
-    };
-    for (uint32_t t = t0; t < t1; t++) count(total_of(t), big_of(t));
+    uint32_t cnt[5] = {0, 0, 0, 0, 0}, s[kPer];
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; u++) {
+        s[u] = tile_seg_log2(n[u], big[u], segLog2, split);
+        count_segments(n[u], s[u], cnt);
+    }
     // the tile-reference prefix rides along as a sixth value
-    uint32_t pos[6] = {cnt[0], cnt[1], cnt[2], cnt[3], cnt[4], localRefs}, tot[6];
-    scan1024_n<6>(pos, sScan6, tot);
-    uint32_t run = pos[5];
+    uint32_t x[6] = {cnt[0], cnt[1], cnt[2], cnt[3], cnt[4], localRefs}, tot6[6];
+    scan1024_n<6>(x, sScan6, tot6);
+    const uint32_t tot[5] = {tot6[0], tot6[1], tot6[2], tot6[3], tot6[4]};
     const uint32_t totalSegs = tot[0] + tot[1] + tot[2] + tot[3] + tot[4];
-    // the thread's image base: segments of all earlier threads' tiles
-    uint32_t seg = pos[0] + pos[1] + pos[2] + pos[3] + pos[4];
-    // list order: full segments, then classes 3, 2, 1, 0
-    pos[4] += tot[0];
-    pos[3] += tot[0] + tot[4];
-    pos[2] += tot[0] + tot[4] + tot[3];
-    pos[1] += tot[0] + tot[4] + tot[3] + tot[2];
     const bool fits = total <= B.ref_cap && totalSegs <= B.work_cap && totalSegs <= kImageMask && segsFit;
-    // A thread's outputs are its contiguous tiles' entries: written straight to
-    // memory, each store instruction touches 64 lines.  Beyond two tiles per
-    // thread they go to LDS instead (a tile's start and item entry over its
-    // total and big count, which only this thread reads) and are copied out
-    // with coalesced stores (10M frame: scans 47 -> 44 us).
-    const bool stageOut = staged && nt > 2048;
-    const bool stageWork = stageOut && totalSegs <= kTilescanWork;
-    uint32_t* sWork = sTiles + 2 * nt;
-    auto place = [&](uint32_t t, uint32_t n, uint32_t big) {
-        if (stageOut) sTiles[t] = run;
-        else B.tile_start[t] = run;
-        run += n;
-        if (fits) {
-            const uint32_t s = tile_log2(n, big, split);
-            const uint32_t nf = n >> s, r = n & ((1u << s) - 1);
-            if (stageOut) sTiles[nt + t] = seg | (s << kImageBits);
-            else B.tile_item[t] = seg | (s << kImageBits);
-            // a tile of one segment is marked (kSingleSegment): its image is
-            // the 32-bit winner orders
-            const uint32_t single = nf + (r ? 1u : 0u) == 1 ? kSingleSegment : 0u;
-            uint32_t* work = stageWork ? sWork : B.work;
-            for (uint32_t i = 0; i < nf; i++) work[pos[0]++] = t | (i << kTileBits) | single;
-            if (r) {
-                const uint32_t c = 1 + (r >> (s - 2));
-                work[pos[c]++] = t | (nf << kTileBits) | single;
-            }
-            seg += nf + (r ? 1u : 0u);
-        }
-    };
-    for (uint32_t t = t0; t < t1; t++) place(t, total_of(t), big_of(t));
-    if (stageOut) {
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < nt; t += 1024) {
-            B.tile_start[t] = sTiles[t];
-            if (fits) B.tile_item[t] = sTiles[nt + t];
-        }
-        if (fits && stageWork)
-            for (uint32_t i = threadIdx.x; i < totalSegs; i += 1024) B.work[i] = sWork[i];
+    // the thread's reference and image base: those of all earlier threads' tiles
+    uint32_t run = x[5], seg = x[0] + x[1] + x[2] + x[3] + x[4], pos[5];
+    class_starts(tot, pos);
+#pragma unroll
+    for (uint32_t c = 0; c < 5; c++) pos[c] += x[c];
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; u++) {
+        const uint32_t t = threadIdx.x * kPer + u;
+        if (t >= nt) break;
+        B.tile_start[t] = run;
+        run += n[u];
+        if (!fits) continue;
+        B.tile_item[t] = seg | (s[u] << kImageBits);
+        seg += place_tile(B.work, t, n[u], s[u], pos);
     }
     if (threadIdx.x == 0) {
         B.tile_start[nt] = total;
@@ -1400,138 +1421,162 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(BatchParams Q, DeviceBuff
     }
 }
 
-// k_bin_tilescan for batches beyond kTilescanStaged tiles, with the same
-// outputs (tile starts, image bases, the same work list in the same order).
-// The three reductions (references and deepest tile; segments with and
-// without the heavy tiles' finer ones; the size classes' totals) stream the
-// counts with coalesced loads.  The placement then takes the tiles in rounds
-// of kTilescanStaged, staged in LDS: each thread takes kRoundPer contiguous
-// tiles of a round, and the six prefixes (five classes, references) carry
-// from round to round.  (Walking a thread's contiguous share of all tiles
-// instead, 113 tiles per thread for 256 jobs, took 0.7 ms: every load
-// instruction touches 64 lines.)
-__global__ __launch_bounds__(1024) void k_bin_tilescan_rounds(BatchParams Q, DeviceBuffers B) {
-    constexpr uint32_t kRound = kTilescanStaged, kRoundPer = kRound / 1024;
-    extern __shared__ uint32_t sTiles[];  // [kRound] totals, then [kRound] big counts
-    __shared__ uint32_t sScan6[6][16];
-    __shared__ uint32_t sRed[4], sCls[5];  // references, deepest, segments, extra; class totals
-    const uint32_t nt = Q.total_tiles;
-    if (threadIdx.x < 4) sRed[threadIdx.x] = 0;
-    if (threadIdx.x < 5) sCls[threadIdx.x] = 0;
-    __syncthreads();
-    uint32_t refs = 0, deepest = 0;
-    for (uint32_t t = threadIdx.x; t < nt; t += 1024) {
-        const uint32_t n = B.tile_totals[t];
-        refs += n;
-        deepest = max(deepest, n);
-    }
-    refs = wave_sum(refs);
-    deepest = wave_max(deepest);
-    if (__lane_id() == 0) {
-        atomicAdd(&sRed[0], refs);
-        atomicMax(&sRed[1], deepest);
-    }
-    __syncthreads();
-    const uint32_t total = sRed[0], maxN = sRed[1];
-    uint32_t segLog2 = kSegLog2Min;
-    while (segLog2 < kSegLog2Max && (total >> segLog2) > B.raster_blocks) segLog2++;
-    while (segLog2 < kSegLog2Max && tile_segments(maxN, segLog2) > (1u << kSegIndexBits)) segLog2++;
-    const bool segsFit = tile_segments(maxN, segLog2) <= (1u << kSegIndexBits);
-    auto tile_log2 = [&](uint32_t n, uint32_t big, bool split) -> uint32_t {
-        if (!split || big < kHeavyBigMin || 4 * big < n) return segLog2;
-        uint32_t s = kSegLog2Heavy;
-        while (s < segLog2 && tile_segments(n, s) > (1u << kSegIndexBits)) s++;
-        return s;
-    };
-    {
-        uint32_t segs = 0, extra = 0;
-        for (uint32_t t = threadIdx.x; t < nt; t += 1024) {
-            const uint32_t n = B.tile_totals[t], big = B.tile_big[t];
-            const uint32_t plain = tile_segments(n, segLog2);
-            segs += plain;
-            extra += tile_segments(n, tile_log2(n, big, true)) - plain;
-        }
-        segs = wave_sum(segs);
-        extra = wave_sum(extra);
-        if (__lane_id() == 0) {
-            atomicAdd(&sRed[2], segs);
-            atomicAdd(&sRed[3], extra);
-        }
-        __syncthreads();
-    }
-    const bool split = (uint64_t)sRed[2] + sRed[3] <= B.work_cap;
-    auto count = [&](uint32_t n, uint32_t big, uint32_t (&cnt)[5]) {
-        const uint32_t s = tile_log2(n, big, split);
-        cnt[0] += n >> s;
-        const uint32_t r = n & ((1u << s) - 1);
-        if (r) cnt[1 + (r >> (s - 2))]++;
-    };
-    {
-        uint32_t cnt[5] = {0, 0, 0, 0, 0};
-        for (uint32_t t = threadIdx.x; t < nt; t += 1024) count(B.tile_totals[t], B.tile_big[t], cnt);
+// The tile scan of more than kTilescanOne tiles.  The references' total and
+// the deepest tile are summed by the column scan already (tile_stats_add), so
+// the segment size is known at once: k_bin_tilesums leaves each block's sums
+// (TileSums), and every block of k_bin_tileplace adds those of the blocks
+// before it and of all (up to 256 blocks: one per thread) and places its own
+// tiles.  Latency bounds both: a block reads 8 KB.  (As one workgroup walking
+// all tiles in rounds of 8,192: 290 us for 117K tiles, 41 us for 16K, 17 us
+// for 8K; the two launches take 12, 11 and 11 us.)
+namespace {
+struct __attribute__((aligned(16))) TileSums {
+    uint32_t refs, segs, extra, pad;  // segments without, and more with, the heavy tiles' finer ones
+    uint32_t plain[5], split[5], pad2[2];  // count_segments without and with them
+};
+static_assert(sizeof(TileSums) == 4 * kTileSumWords, "TileSums layout");
+constexpr uint32_t kTilePer = kTileBlock / kBlock;
+static_assert(kTilePer == 4, "a thread's tiles are one 16-byte load");
+static_assert(kMaxBatchTiles / kTileBlock <= kBlock, "k_bin_tileplace takes one block's sums per thread");
+
+__device__ __forceinline__ uint32_t tile_stats_total(const DeviceBuffers& B, uint32_t& deepest) {
+    uint32_t total = 0;
+    deepest = 0;
 #pragma unroll
-        for (int c = 0; c < 5; c++) {
-            const uint32_t v = wave_sum(cnt[c]);
-            if (__lane_id() == 0 && v) atomicAdd(&sCls[c], v);
-        }
-        __syncthreads();
+    for (uint32_t k = 0; k < kAllocStripes; k++) {
+        total += B.counters[kCntTileRefs + k];
+        deepest = max(deepest, B.counters[kCntTileDeepest + k]);
     }
-    const uint32_t totalSegs = sCls[0] + sCls[1] + sCls[2] + sCls[3] + sCls[4];
+    return total;
+}
+
+// The thread's kTilePer tiles (totals and big counts; 0 beyond the last).
+__device__ __forceinline__ void load_tiles(const BatchParams& Q, const DeviceBuffers& B, uint32_t t0,
+                                           uint32_t (&n)[kTilePer], uint32_t (&big)[kTilePer]) {
+    if (t0 + kTilePer <= Q.total_tiles) {
+        const uint4 a = *reinterpret_cast<const uint4*>(B.tile_totals + t0);
+        const uint4 b = *reinterpret_cast<const uint4*>(B.tile_big + t0);
+        n[0] = a.x; n[1] = a.y; n[2] = a.z; n[3] = a.w;
+        big[0] = b.x; big[1] = b.y; big[2] = b.z; big[3] = b.w;
+    } else {
+#pragma unroll
+        for (uint32_t u = 0; u < kTilePer; u++) {
+            n[u] = t0 + u < Q.total_tiles ? B.tile_totals[t0 + u] : 0u;
+            big[u] = t0 + u < Q.total_tiles ? B.tile_big[t0 + u] : 0u;
+        }
+    }
+}
+}  // namespace
+
+__global__ __launch_bounds__(kBlock) void k_bin_tilesums(BatchParams Q, DeviceBuffers B) {
+    __shared__ uint32_t sSum[13];
+    if (threadIdx.x < 13) sSum[threadIdx.x] = 0;
+    uint32_t n[kTilePer], big[kTilePer], deepest;
+    load_tiles(Q, B, (blockIdx.x * kBlock + threadIdx.x) * kTilePer, n, big);
+    const uint32_t total = tile_stats_total(B, deepest);
+    bool segsFit;
+    const uint32_t segLog2 = frame_seg_log2(total, deepest, B.raster_blocks, segsFit);
+    uint32_t plain[5] = {0, 0, 0, 0, 0}, split[5] = {0, 0, 0, 0, 0}, refs = 0, segs = 0, extra = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kTilePer; u++) {
+        const uint32_t s = tile_seg_log2(n[u], big[u], segLog2, true);
+        const uint32_t p = tile_segments(n[u], segLog2);
+        refs += n[u];
+        segs += p;
+        extra += tile_segments(n[u], s) - p;
+        count_segments(n[u], segLog2, plain);
+        count_segments(n[u], s, split);
+    }
+    const uint32_t v[13] = {refs, segs, extra, plain[0], plain[1], plain[2], plain[3], plain[4],
+                            split[0], split[1], split[2], split[3], split[4]};
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 13; k++) {
+        const uint32_t w = wave_sum(v[k]);
+        if (__lane_id() == 0 && w) atomicAdd(&sSum[k], w);
+    }
+    __syncthreads();
+    if (threadIdx.x < 13)  // (the struct's words, past its pad)
+        B.tile_sums[blockIdx.x * kTileSumWords + threadIdx.x + (threadIdx.x >= 3 ? 1u : 0u)] = sSum[threadIdx.x];
+}
+
+__global__ __launch_bounds__(kBlock) void k_bin_tileplace(BatchParams Q, DeviceBuffers B) {
+    constexpr uint32_t kWaves = kBlock / kWave;
+    __shared__ uint32_t sAll[kWaves][8], sBefore[kWaves][6], sScan[kWaves][6];
+    const uint32_t lane = __lane_id(), wave = threadIdx.x / kWave, nb = gridDim.x;
+    const uint32_t t0 = (blockIdx.x * kBlock + threadIdx.x) * kTilePer;
+    uint32_t n[kTilePer], big[kTilePer], deepest;
+    load_tiles(Q, B, t0, n, big);
+    TileSums sums;
+    memset(&sums, 0, sizeof(sums));
+    if (threadIdx.x < nb) sums = reinterpret_cast<const TileSums*>(B.tile_sums)[threadIdx.x];
+    const uint32_t total = tile_stats_total(B, deepest);
+    bool segsFit;
+    const uint32_t segLog2 = frame_seg_log2(total, deepest, B.raster_blocks, segsFit);
+    // The finer segments of heavy tiles are taken only while the work list has room for them.
+    const uint32_t ws = wave_sum(sums.segs), we = wave_sum(sums.extra);
+    if (lane == 0) {
+        sAll[wave][5] = ws;
+        sAll[wave][6] = we;
+    }
+    __syncthreads();
+    uint64_t want = 0;
+    for (uint32_t w = 0; w < kWaves; w++) want += (uint64_t)sAll[w][5] + sAll[w][6];
+    const bool split = want <= B.work_cap;
+    // all blocks' classes, and the classes and references of the blocks before this one
+    const bool before = threadIdx.x < blockIdx.x;
+#pragma unroll
+    for (int c = 0; c < 5; c++) {
+        const uint32_t v = split ? sums.split[c] : sums.plain[c];
+        const uint32_t a = wave_sum(v), b = wave_sum(before ? v : 0u);
+        if (lane == 0) {
+            sAll[wave][c] = a;
+            sBefore[wave][c] = b;
+        }
+    }
+    const uint32_t rb = wave_sum(before ? sums.refs : 0u);
+    if (lane == 0) sBefore[wave][5] = rb;
+    // this block's own scan of the same six
+    uint32_t cnt[5] = {0, 0, 0, 0, 0}, s[kTilePer], refs = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kTilePer; u++) {
+        s[u] = tile_seg_log2(n[u], big[u], segLog2, split);
+        count_segments(n[u], s[u], cnt);
+        refs += n[u];
+    }
+    uint32_t x[6] = {cnt[0], cnt[1], cnt[2], cnt[3], cnt[4], refs};
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+        const uint32_t incl = wave_incl_scan(x[c]);
+        if (lane == kWave - 1) sScan[wave][c] = incl;
+        x[c] = incl - x[c];
+    }
+    __syncthreads();
+    uint32_t tot[5] = {0, 0, 0, 0, 0};
+    for (uint32_t w = 0; w < kWaves; w++) {
+#pragma unroll
+        for (int c = 0; c < 6; c++) x[c] += sBefore[w][c] + (w < wave ? sScan[w][c] : 0u);
+#pragma unroll
+        for (int c = 0; c < 5; c++) tot[c] += sAll[w][c];
+    }
+    const uint32_t totalSegs = tot[0] + tot[1] + tot[2] + tot[3] + tot[4];
     const bool fits = total <= B.ref_cap && totalSegs <= B.work_cap && totalSegs <= kImageMask && segsFit;
-    // list order: full segments, then classes 3, 2, 1, 0
-    uint32_t pos[5] = {0, sCls[0] + sCls[4] + sCls[3] + sCls[2], sCls[0] + sCls[4] + sCls[3], sCls[0] + sCls[4],
-                       sCls[0]};
-    uint32_t run = 0, seg = 0;  // references and segments of the earlier rounds
-    for (uint32_t r0 = 0; r0 < nt; r0 += kRound) {
-        const uint32_t rn = min(kRound, nt - r0);
-        __syncthreads();  // the previous round's LDS entries are copied out
-        for (uint32_t i = threadIdx.x; i < rn; i += 1024) {
-            sTiles[i] = B.tile_totals[r0 + i];
-            sTiles[kRound + i] = B.tile_big[r0 + i];
-        }
-        __syncthreads();
-        const uint32_t a0 = min(rn, threadIdx.x * kRoundPer), a1 = min(rn, a0 + kRoundPer);
-        uint32_t cnt[5] = {0, 0, 0, 0, 0}, mine = 0;
-        for (uint32_t i = a0; i < a1; i++) {
-            mine += sTiles[i];
-            count(sTiles[i], sTiles[kRound + i], cnt);
-        }
-        uint32_t x[6] = {cnt[0], cnt[1], cnt[2], cnt[3], cnt[4], mine}, tot[6];
-        scan1024_n<6>(x, sScan6, tot);
-        uint32_t p[5], tRun = run + x[5], tSeg = seg + x[0] + x[1] + x[2] + x[3] + x[4];
+    uint32_t run = x[5], seg = x[0] + x[1] + x[2] + x[3] + x[4], pos[5];
+    class_starts(tot, pos);
 #pragma unroll
-        for (int c = 0; c < 5; c++) p[c] = pos[c] + x[c];
-        // a tile's start and item entry over its total and big count, which
-        // only this thread reads; copied out with coalesced stores below
-        for (uint32_t i = a0; i < a1; i++) {
-            const uint32_t t = r0 + i, n = sTiles[i], big = sTiles[kRound + i];
-            sTiles[i] = tRun;
-            tRun += n;
-            if (fits) {
-                const uint32_t s = tile_log2(n, big, split);
-                const uint32_t nf = n >> s, r = n & ((1u << s) - 1);
-                sTiles[kRound + i] = tSeg | (s << kImageBits);
-                const uint32_t single = nf + (r ? 1u : 0u) == 1 ? kSingleSegment : 0u;
-                for (uint32_t k = 0; k < nf; k++) B.work[p[0]++] = t | (k << kTileBits) | single;
-                if (r) {
-                    const uint32_t c = 1 + (r >> (s - 2));
-                    B.work[p[c]++] = t | (nf << kTileBits) | single;
-                }
-                tSeg += nf + (r ? 1u : 0u);
-            }
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < rn; i += 1024) {
-            B.tile_start[r0 + i] = sTiles[i];
-            if (fits) B.tile_item[r0 + i] = sTiles[kRound + i];
-        }
+    for (int c = 0; c < 5; c++) pos[c] += x[c];
 #pragma unroll
-        for (int c = 0; c < 5; c++) pos[c] += tot[c];
-        run += tot[5];
-        seg += tot[0] + tot[1] + tot[2] + tot[3] + tot[4];
+    for (uint32_t u = 0; u < kTilePer; u++) {
+        const uint32_t t = t0 + u;
+        if (t >= Q.total_tiles) break;
+        B.tile_start[t] = run;
+        run += n[u];
+        if (!fits) continue;
+        B.tile_item[t] = seg | (s[u] << kImageBits);
+        seg += place_tile(B.work, t, n[u], s[u], pos);
     }
-    if (threadIdx.x == 0) {
-        B.tile_start[nt] = total;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        B.tile_start[Q.total_tiles] = total;
         B.counters[kCntTotalRefs] = total;
         B.counters[kCntWorkItems] = totalSegs;
         B.counters[kCntSegLog2] = segLog2;
@@ -2573,12 +2618,6 @@ hipError_t init_kernels() {
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void*)k_bin_scatter, hipFuncAttributeMaxDynamicSharedMemorySize, maxDyn);
     if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)k_bin_tilescan, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(uint32_t) * (2 * kTilescanStaged + kTilescanWork)));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)k_bin_tilescan_rounds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(uint32_t) * 2 * kTilescanStaged));
-    if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&g_rasterResident[0],
                                                          reinterpret_cast<const void*>(&k_raster<false>), kBlock, 0);
     if (e == hipSuccess)
@@ -2683,12 +2722,15 @@ hipError_t launch_frame(const BatchParams& Q, FrameParams* jobs, const FramePara
         const dim3 passGrid(colGrid.x, max(1u, colGrid.y), colGrid.z);
         hipLaunchKernelGGL(k_bin_colpass, passGrid, dim3(kBlock), 0, s, Q, jobs, B);
     }
-    if (Q.total_tiles <= kTilescanStaged)
-        hipLaunchKernelGGL(k_bin_tilescan, dim3(1), dim3(1024),
-                           sizeof(uint32_t) * (2 * (size_t)Q.total_tiles + kTilescanWork), s, Q, B);
-    else
-        hipLaunchKernelGGL(k_bin_tilescan_rounds, dim3(1), dim3(1024), sizeof(uint32_t) * 2 * kTilescanStaged, s, Q,
-                           B);
+    if (Q.total_tiles <= kTilescanOne) {
+        if (Q.total_tiles <= 1024) hipLaunchKernelGGL(k_bin_tilescan<1>, dim3(1), dim3(1024), 0, s, Q, B);
+        else if (Q.total_tiles <= 2048) hipLaunchKernelGGL(k_bin_tilescan<2>, dim3(1), dim3(1024), 0, s, Q, B);
+        else hipLaunchKernelGGL(k_bin_tilescan<4>, dim3(1), dim3(1024), 0, s, Q, B);
+    } else {
+        const dim3 blocks((Q.total_tiles + kTileBlock - 1) / kTileBlock);
+        hipLaunchKernelGGL(k_bin_tilesums, blocks, dim3(kBlock), 0, s, Q, B);
+        hipLaunchKernelGGL(k_bin_tileplace, blocks, dim3(kBlock), 0, s, Q, B);
+    }
     mark(3);
     if (Q.total_chunks) hipLaunchKernelGGL(k_bin_scatter, dim3(Q.total_chunks), dim3(kBlock), lds, s, Q, jobs, B);
     mark(4);
