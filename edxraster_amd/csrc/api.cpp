@@ -786,7 +786,7 @@ int edxr_create(edxr_ctx** out, uint32_t width, uint32_t height) {
     // address is looked up here, once per device, never in a render call.
     if (e == hipSuccess) e = scratch_address(&c->scratch);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    // coherent: the frame's last kernel writes it, the host reads it after a stream synchronisation
+    // coherent: k_raster writes it, the host reads it after a stream synchronisation
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->hostCounters, sizeof(uint32_t) * kCntSlots, hipHostMallocCoherent);
     if (e == hipSuccess) e = c->counters.ensure(kCntSlots);
     if (e == hipSuccess) {

@@ -167,15 +167,6 @@ __global__ void k_reset(uint32_t* counters, FrameParams* jobs, FrameParams job0,
     if (writeJob && threadIdx.x == 0) jobs[0] = job0;
 }
 
-// The frame's last launch: the counters to the host's pinned buffer, which
-// the host reads once the stream has drained (no copy queued behind the
-// frame, whose start would wait for the frame's end and then for its own
-// launch).
-__global__ void k_publish(const uint32_t* counters, uint32_t* host) {
-    for (uint32_t i = threadIdx.x; i < kCntSlots; i += blockDim.x) host[i] = counters[i];
-    __threadfence_system();
-}
-
 
 // Sample offsets in 28.4 units per MSAA level, (x, y) per sample: the table of
 // FrameBuffer::MultiSampleOffsets (Core/FrameBuffer.cpp:107-191).
@@ -2388,6 +2379,14 @@ __global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, c
     __shared__ uint64_t keys[(kMS ? kPassSamples : 1) * kKeyPlane<kMS>];
     __shared__ uint16_t sOwner[kBlock / kWave][kOwnerCap];
     __shared__ uint32_t sItem;
+    // The counters are final (this kernel only draws items from kCntWorkNext):
+    // the last workgroup, which in small frames has no item, copies them to
+    // the host's pinned buffer, which the host reads once the stream has
+    // drained.  The stores are on their way while the frame is rasterised; a
+    // launch of its own after the frame took 4 us and the gap before it, and
+    // a copy queued behind the frame 12 us.
+    if (blockIdx.x == gridDim.x - 1)
+        for (uint32_t i = threadIdx.x; i < kCntSlots; i += kBlock) B.host_counters[i] = B.counters[i];
     if (B.counters[kCntOverflow] & kOvNoLists) return;
     const uint32_t nItems = B.counters[kCntWorkItems];
     // Single-sample batches: the empty tiles are cleared here, a share per
@@ -2739,7 +2738,6 @@ hipError_t launch_frame(const BatchParams& Q, FrameParams* jobs, const FramePara
     if (Q.any_textured) hipLaunchKernelGGL(k_shade_tex, dim3(2 * Q.total_tiles), dim3(512), 0, s, Q, jobs, B);
     else hipLaunchKernelGGL(k_shade, dim3(2 * Q.total_tiles), dim3(512), 0, s, Q, jobs, B);
     mark(5);
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(256), 0, s, B.counters, B.host_counters);
     return hipGetLastError();
 }
 
