@@ -218,6 +218,16 @@ struct edxr_ctx {
     // The one-pass column scan gave up waiting once (or debug capacities make
     // it give up at once): three-kernel column scans from then on.
     bool legacyScans = false;
+    // Direct frames (k_front): their counters and the tiles' count words, zero
+    // between frames (directDirty: a frame was launched and not seen to end).
+    // A frame with a tile too deep for them is run again on the general path,
+    // which then takes the next directSkip frames: twice as many after each
+    // such frame, half as many after each that went well.
+    DevBuf<uint32_t> directCounters;
+    DevBuf<uint64_t> tileCount;
+    bool directDirty = true;
+    uint32_t lastDirect = 0;        // list entries per tile of the last frame, if it was a direct one
+    uint32_t directSkip = 0, directBackoff = 0;
     uint8_t* scratch = nullptr;     // device address of this device's no-allocation scratch
     uint64_t renderGeneration = 0;  // advanced by every render_mesh / render_batch
     uint32_t* hostCounters = nullptr;
@@ -464,6 +474,65 @@ void drop_graph(edxr_ctx* c) {
     c->graphKey.clear();
 }
 
+// Whether a frame is launched as a direct one (k_front): where its fewer
+// launches save more than the general path's better split of deep tiles does.
+// Measured, general and direct: 4,096-triangle sphere at 800x600 72 and 34 us,
+// 360K-triangle sphere at 1080p 84 and 58, 498K heightfield at 1080p 113 and
+// 90, 819K sphere grid at 1080p 143 and 118, 1M sphere at 4K 138 and 105, 128
+// jobs of up to 20K at 513^2 316 and 259; beyond a million triangles 226 and
+// 233 (2M heightfield at 4K), 157 and 159 (2M sphere grid), 382 and 389 (60
+// jobs of up to 100K at 1024^2).  With more than kDirectSlots triangles per
+// tile the deepest tiles mostly exceed a list (179K heightfield at 640x480).
+// Not with capacities or chunks set by the caller, which are the general
+// path's.
+bool direct_frame(edxr_ctx* c, const BatchParams& Q) {
+    if (Q.max_samples != 1 || !Q.total_slots || Q.total_tiles > kDirectMaxTiles ||
+        Q.total_slots > kDirectMaxSlots || c->debugCapacity || (Q.num_jobs == 1 && c->binChunksSetting) ||
+        (uint64_t)Q.total_slots > (uint64_t)kDirectSlots * Q.total_tiles)
+        return false;
+    if (!c->directSkip) return true;
+    c->directSkip--;
+    return false;
+}
+
+// Entries of a direct frame's tile lists.
+uint32_t direct_cap(const BatchParams& Q) { return Q.total_tiles <= kDirectFewTiles ? kDirectCap : kDirectCapMany; }
+
+// Gives the buffers of a direct frame their counters and count words, cleared
+// where an earlier frame may not have done so.
+hipError_t direct_begin(edxr_ctx* c, DeviceBuffers& B, uint32_t cap) {
+    if (c->directDirty) {
+        hipError_t e = hipMemsetAsync(c->directCounters.p, 0, sizeof(uint32_t) * kCntSlots, c->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(c->tileCount.p, 0, sizeof(uint64_t) * kDirectMaxTiles, c->stream);
+        if (e != hipSuccess) return e;
+    }
+    B.direct = cap;
+    B.counters = c->directCounters.p;
+    B.tile_count = c->tileCount.p;
+    c->directDirty = true;
+    return hipSuccess;
+}
+
+// After a direct frame has ended: whether it has to be run again on the general path.
+bool direct_end(edxr_ctx* c, uint32_t overflow) {
+    c->directDirty = false;
+    if (!(overflow & kOvDirect)) {
+        c->directBackoff /= 2;
+        return false;
+    }
+    c->directBackoff = std::min(1024u, std::max(16u, 2 * c->directBackoff));
+    c->directSkip = c->directBackoff;
+    return true;
+}
+
+// References of a frame's tiles (h: the counters read back).
+uint32_t total_refs(const uint32_t* h, bool direct) {
+    if (!direct) return h[kCntTotalRefs];
+    uint32_t n = 0;
+    for (uint32_t k = 0; k < kAllocStripes; k++) n += h[kCntTileRefs + k];
+    return n;
+}
+
 // Runs a planned batch (sized, launched, checked; re-run with larger buffers
 // after a capacity overflow).  For a single job the job table is written by
 // the frame's first kernel, which takes the job by value (in a graph replay,
@@ -473,7 +542,6 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
     hipError_t e;
     BatchParams& Q = pl.Q;
     const bool single = Q.num_jobs == 1;
-    const bool graph = c->useGraph != 0;
     if ((e = c->jobsDev.ensure(Q.num_jobs)) != hipSuccess ||
         (e = c->tileTotals.ensure(Q.total_tiles)) != hipSuccess ||
         (e = c->tileStart.ensure((size_t)Q.total_tiles + 1)) != hipSuccess ||
@@ -517,21 +585,25 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
     // Raster work items per frame the segment size aims for (tuning).
     const uint32_t rasterBlocks = c->numCUs * (c->rasterPerCU ? c->rasterPerCU : 8);
     c->stats = edxr_stats{};
-    for (uint32_t attempt = 0; attempt < 8; attempt++) {
+    bool direct = direct_frame(c, Q);
+    for (uint32_t attempt = 0; attempt < 8;) {
         if ((uint64_t)T + c->extraRecCap > kRecordMask) return c->fail(EDXR_E_LIMIT, "record capacity exceeded");
         if ((e = c->rrec.ensure((size_t)T + c->extraRecCap)) != hipSuccess ||
             (e = c->srec.ensure((size_t)T + c->extraRecCap)) != hipSuccess ||
             (e = c->desc.ensure(std::max<uint32_t>(T, 1))) != hipSuccess ||
-            (e = c->chunkBox.ensure(2 * std::max<uint32_t>(Q.total_chunks, 1))) != hipSuccess ||
-            (e = c->groupSums.ensure(std::max<uint64_t>(pl.groupEntries, 1))) != hipSuccess ||
             (e = c->clipQueue.ensure(c->clipQueueCap)) != hipSuccess ||
-            (e = c->binCounts.ensure(std::max<uint64_t>(pl.countEntries, 1))) != hipSuccess ||
-            (e = c->refs.ensure(c->refCap)) != hipSuccess ||
-            (e = c->work.ensure((size_t)Q.total_tiles + std::max(rasterBlocks, c->refCap / kSegRefs) + 2)) !=
-                hipSuccess ||
-            (e = c->partials.ensure(c->work.cap * kTileSize * kTileSize * Q.max_samples)) != hipSuccess ||
+            (e = c->refs.ensure(direct ? std::max((size_t)c->refCap, (size_t)Q.total_tiles * direct_cap(Q))
+                                       : (size_t)c->refCap)) != hipSuccess ||
             (e = c->verts.ensure((size_t)V + c->extraVertCap)) != hipSuccess ||
             (e = c->sverts.ensure(std::max<uint32_t>(V, 1))) != hipSuccess)
+            return c->hip_fail(e, "hipMalloc(pipeline)");
+        if (!direct &&
+            ((e = c->chunkBox.ensure(2 * std::max<uint32_t>(Q.total_chunks, 1))) != hipSuccess ||
+             (e = c->groupSums.ensure(std::max<uint64_t>(pl.groupEntries, 1))) != hipSuccess ||
+             (e = c->binCounts.ensure(std::max<uint64_t>(pl.countEntries, 1))) != hipSuccess ||
+             (e = c->work.ensure((size_t)Q.total_tiles + std::max(rasterBlocks, c->refCap / kSegRefs) + 2)) !=
+                 hipSuccess ||
+             (e = c->partials.ensure(c->work.cap * kTileSize * kTileSize * Q.max_samples)) != hipSuccess))
             return c->hip_fail(e, "hipMalloc(pipeline)");
 
         // Zeroed as a whole: the structure's bytes, padding included, are
@@ -576,8 +648,12 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
         B.depth = depth;
         B.ids = ids;
         B.color_f32 = colorF;
+        if (direct && (e = direct_begin(c, B, direct_cap(Q))) != hipSuccess) return c->hip_fail(e, "hipMemsetAsync(direct frame)");
 
-        const bool prof = c->profile && !graph;
+        // Three launches cost the host less than a graph's: 4,096-triangle
+        // sphere 34 us eager, 40 us replayed.
+        const bool graph = c->useGraph != 0 && !direct;
+        const bool prof = c->profile && !c->useGraph;
         if (graph) {
             const std::vector<uint8_t> key = launch_key(Q, B, c->jobsDev.p);
             const FrameParams* job0 = single ? &pl.jobs[0] : nullptr;
@@ -617,10 +693,12 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
         if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return c->hip_fail(e, "hipStreamSynchronize");
         const uint32_t* h = c->hostCounters;
         const uint32_t ov = h[kCntOverflow];
+        const bool toGeneral = direct && direct_end(c, ov);
         if (ov & kOvPolygon) return c->fail(EDXR_E_LIMIT, "clip polygon exceeded 9 vertices");
         if (!ov) {
             if (h[kCntBadIndex])
                 return c->fail(EDXR_E_INDEX, "triangle index >= num_vertices or texture slot >= texture count");
+            c->lastDirect = B.direct;
             uint64_t tin = 0;
             for (const FrameParams& P : pl.jobs) tin += P.num_triangles;
             const CounterSums cs = counter_sums(h);
@@ -629,7 +707,7 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
             c->stats.clipped = cs.clipped;
             c->stats.near_clipped = cs.nearClipped;
             c->stats.setup_records = cs.mainRecords + cs.extraRecs;
-            c->stats.refs = h[kCntTotalRefs];
+            c->stats.refs = total_refs(h, direct);
             c->stats.clip_vertices = cs.extraVerts;
             c->stats.retries = attempt;
             c->stats.bin_chunks = Q.total_chunks;
@@ -656,7 +734,10 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
             c->extraRecCap = std::max(c->extraRecCap, grow(2 * c->extraRecCap));
             c->extraVertCap = std::max(c->extraVertCap, grow(2 * c->extraVertCap));
         }
-        c->stats.retries = attempt + 1;
+        // (the step to the general path is no capacity retry)
+        if (toGeneral) direct = false;
+        else attempt++;
+        c->stats.retries = attempt;
     }
     return c->fail(EDXR_E_LIMIT, "capacity retries exhausted");
 }
@@ -789,6 +870,8 @@ int edxr_create(edxr_ctx** out, uint32_t width, uint32_t height) {
     // coherent: k_raster writes it, the host reads it after a stream synchronisation
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->hostCounters, sizeof(uint32_t) * kCntSlots, hipHostMallocCoherent);
     if (e == hipSuccess) e = c->counters.ensure(kCntSlots);
+    if (e == hipSuccess) e = c->directCounters.ensure(kCntSlots);
+    if (e == hipSuccess) e = c->tileCount.ensure(kDirectMaxTiles);
     if (e == hipSuccess) {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0)
@@ -820,7 +903,7 @@ void edxr_destroy(edxr_ctx* c) {
     c->rrec.release();
     c->srec.release();
     for (DevBuf<uint32_t>* b : {&c->desc, &c->clipQueue, &c->binCounts, &c->tileTotals, &c->tileStart, &c->refs,
-                                &c->counters, &c->color, &c->ids, &c->work, &c->tileItem, &c->tileBig, &c->tileSums, &c->groupSums,
+                                &c->counters, &c->directCounters, &c->color, &c->ids, &c->work, &c->tileItem, &c->tileBig, &c->tileSums, &c->groupSums,
                                 &c->jobTables, &c->bcolor, &c->bids})
         b->release();
     c->depth.release();
@@ -832,6 +915,7 @@ void edxr_destroy(edxr_ctx* c) {
     c->adjAcc.release();
     c->adjVertAcc.release();
     c->partials.release();
+    c->tileCount.release();
     c->chunkBox.release();
     c->verts.release();
     c->sverts.release();
@@ -1044,7 +1128,8 @@ int edxr_render_mesh_noalloc(edxr_ctx* c, const edxr_mesh* m, void* color, void*
     bool legacyScans = c->legacyScans;
     hipError_t e;
     c->stats = edxr_stats{};
-    for (uint32_t attempt = 0; attempt < 8; attempt++) {
+    bool direct = direct_frame(c, Q);
+    for (uint32_t attempt = 0; attempt < 8;) {
         if ((uint64_t)T + recCap > kRecordMask) return c->fail(EDXR_E_LIMIT, "record capacity exceeded");
         const uint64_t workCap = (uint64_t)P.num_tiles + std::max(rasterBlocks, refCap / kSegRefs) + 2;
         ScratchCarver s{c->scratch};
@@ -1095,11 +1180,18 @@ int edxr_render_mesh_noalloc(edxr_ctx* c, const edxr_mesh* m, void* color, void*
         B.depth = static_cast<float*>(depth);
         B.ids = static_cast<uint32_t*>(ids);
         B.color_f32 = nullptr;
+        if (direct) {
+            // the key images' place (8 KB per tile and more), which a direct frame does not use
+            static_assert(kDirectCapMany * sizeof(uint32_t) <= kTileSize * kTileSize * sizeof(uint64_t), "a tile's list");
+            B.refs = reinterpret_cast<uint32_t*>(B.partials);
+            if ((e = direct_begin(c, B, kDirectCapMany)) != hipSuccess) return c->hip_fail(e, "hipMemsetAsync(direct frame)");
+        }
         // The first kernel writes the job table from its argument: no upload.
         if ((e = launch_frame(Q, jobs, &P, B, c->stream, nullptr)) != hipSuccess) return c->hip_fail(e, "kernel launch");
         if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return c->hip_fail(e, "hipStreamSynchronize");
         const uint32_t* h = c->hostCounters;
         const uint32_t ov = h[kCntOverflow];
+        const bool toGeneral = direct && direct_end(c, ov);
         if (ov & kOvPolygon) return c->fail(EDXR_E_LIMIT, "clip polygon exceeded 9 vertices");
         if (!ov) {
             if (h[kCntBadIndex])
@@ -1110,7 +1202,7 @@ int edxr_render_mesh_noalloc(edxr_ctx* c, const edxr_mesh* m, void* color, void*
             c->stats.clipped = cs.clipped;
             c->stats.near_clipped = cs.nearClipped;
             c->stats.setup_records = cs.mainRecords + cs.extraRecs;
-            c->stats.refs = h[kCntTotalRefs];
+            c->stats.refs = total_refs(h, direct);
             c->stats.clip_vertices = cs.extraVerts;
             c->stats.retries = attempt;
             c->stats.bin_chunks = P.num_chunks;
@@ -1129,6 +1221,8 @@ int edxr_render_mesh_noalloc(edxr_ctx* c, const edxr_mesh* m, void* color, void*
         if (ov & kOvExtraVertices) vertCap = grow(std::max(cs.vertDemand, 2 * vertCap));
         if (ov & kOvRefs) refCap = grow(std::max(h[kCntTotalRefs], refCap));
         if (ov & kOvScanWait) legacyScans = c->legacyScans = true;
+        if (toGeneral) direct = false;
+        else attempt++;
     }
     return c->fail(EDXR_E_LIMIT, "capacity retries exhausted");
 }
@@ -1585,12 +1679,28 @@ int64_t edxr_debug_read_bins(edxr_ctx* c, uint64_t* offsets, uint32_t* refs3, ui
     std::vector<uint32_t> ts(c->nTiles + 1);
     hipError_t e = hipMemcpy(ts.data(), c->tileStart.p, 4ull * (c->nTiles + 1), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return c->hip_fail(e, "debug_read_bins");
+    if (c->lastDirect) {  // the tiles' counts
+        uint32_t run = 0;
+        for (uint32_t i = 0; i < c->nTiles; i++) {
+            const uint32_t n = ts[i];
+            ts[i] = run;
+            run += n;
+        }
+        ts[c->nTiles] = run;
+    }
     const uint64_t total = ts[c->nTiles];
     std::vector<uint32_t> refs(total);
     const uint64_t nrec = (uint64_t)c->lastT + c->extraRecCap;
     std::vector<RasterRec> rr(nrec);
     std::vector<ShadeRec> sr(nrec);
-    if (total) e = hipMemcpy(refs.data(), c->refs.p, 4ull * total, hipMemcpyDeviceToHost);
+    if (total && c->lastDirect) {
+        std::vector<uint32_t> all((size_t)c->nTiles * c->lastDirect);
+        e = hipMemcpy(all.data(), c->refs.p, 4ull * all.size(), hipMemcpyDeviceToHost);
+        for (uint32_t i = 0; i < c->nTiles; i++)
+            std::copy_n(&all[(size_t)i * c->lastDirect], ts[i + 1] - ts[i], refs.begin() + ts[i]);
+    } else if (total) {
+        e = hipMemcpy(refs.data(), c->refs.p, 4ull * total, hipMemcpyDeviceToHost);
+    }
     if (e == hipSuccess) e = hipMemcpy(rr.data(), c->rrec.p, sizeof(RasterRec) * nrec, hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(sr.data(), c->srec.p, sizeof(ShadeRec) * nrec, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return c->hip_fail(e, "debug_read_bins");

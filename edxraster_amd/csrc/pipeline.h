@@ -39,6 +39,18 @@ constexpr uint32_t kChunkGroup = 64;         // chunks per block of the column s
 constexpr uint32_t kTilescanOne = 4096;
 constexpr uint32_t kTileBlock = 1024;        // tiles per workgroup of the two launches
 constexpr uint32_t kTileSumWords = 16;       // words of a workgroup's sums between them
+// Direct frames (k_front): entries of a tile's list, and tile-level references
+// among them that one workgroup walks; a tile beyond either sends the frame to
+// the general path, which cuts such tiles into segments.  The lists take 16 KB
+// a tile, 8 KB beyond kDirectFewTiles, where the general path's key images take
+// 8 KB, and as much in the place of those in the allocation-free frame.
+constexpr uint32_t kDirectCap = 4096;
+constexpr uint32_t kDirectCapMany = 2048;
+constexpr uint32_t kDirectFewTiles = 8192;
+constexpr uint32_t kDirectHeavy = 48;
+constexpr uint32_t kDirectMaxTiles = 32768;
+constexpr uint32_t kDirectMaxSlots = 1u << 20;  // triangle slots of a direct frame,
+constexpr uint32_t kDirectSlots = 512;          // and per tile on average, at most
 constexpr uint32_t kScanSpinLimit = 1u << 20;  // k_bin_colpass look-back waits (about 30 ms) before giving up
 // Single-sample shading rebuilds a winner's screen values from its shading
 // vertices, instead of gathering them, in tiles of this many references or
@@ -214,7 +226,7 @@ enum CounterSlot {
     kCntStriped = 16,    // high-rate counters: kStripes slots each, summed on the host
     kCntAllocStriped = kCntStriped + 4 * 32,  // k_clip's allocations: kAllocStripes vertices, then records
     kCntTileRefs = kCntAllocStriped + 2 * 16,  // tile references and deepest tile, kAllocStripes each
-    kCntTileDeepest = kCntTileRefs + 16,       // (frames of more than kTilescanOne tiles)
+    kCntTileDeepest = kCntTileRefs + 16,       // (frames of more than kTilescanOne tiles; references of direct frames)
     kCntSlots = kCntTileDeepest + 16
 };
 
@@ -232,6 +244,7 @@ enum OverflowBit {
     kOvExtraVertices = 4,
     kOvRefs = 8,
     kOvPolygon = 16,
+    kOvDirect = 64,      // a direct frame has a tile for the general path: re-run there
     kOvScanWait = 32     // a k_bin_colpass look-back gave up waiting: re-run with the three-kernel scan
 };
 // Overflows after which the tile lists are not valid: the scatter, raster
@@ -257,12 +270,11 @@ struct DeviceBuffers {
     uint32_t legacy_scans;     // 1: column sums, group scan and column scan as three kernels
     uint32_t* tile_totals;
     uint32_t* tile_start;  // num_tiles + 1
-    uint32_t* refs;
+    uint32_t* refs;        // (direct frames: `direct` entries per tile)
     uint32_t ref_cap;
     uint32_t* work;        // raster work items: global tile | segment << kTileBits | kSingleSegment
     uint32_t work_cap;
     uint32_t* tile_item;   // per global tile: first key image (one per segment) | segment log2 << kImageBits
-    uint32_t* tile_sums;   // kTileSumWords per kTileBlock tiles (frames of more than kTilescanOne tiles)
     uint32_t* tile_big;    // per global tile: heavy references (big, or compact with kDescHeavy)
     uint64_t* partials;    // work_cap * samples * 1024 (depth, order) keys, one tile image per item and sample
     uint32_t raster_blocks;  // work items the segment size is chosen for
@@ -274,6 +286,9 @@ struct DeviceBuffers {
     float* depth;          // samples planes of the job's pixels (single frame), sample-major
     uint32_t* ids;
     float* color_f32;      // optional clamped float RGB (3 per pixel) for the adjoint
+    uint32_t* tile_sums;   // kTileSumWords per kTileBlock tiles (frames of more than kTilescanOne tiles)
+    uint64_t* tile_count;  // direct frames, per tile: references | heavy references << 32; zero between frames
+    uint32_t direct;       // entries of a tile's list; 0: not a direct frame
 };
 
 // Gradient outputs of one job (device pointers, accumulated with +=; any may
@@ -317,6 +332,11 @@ hipError_t launch_adjoint(const BatchParams& Q, const FrameParams* jobs, const G
                           double* vacc, uint64_t vacc_size, bool any_pow, hipStream_t s);
 // Kernel attributes (dynamic LDS limits) and occupancy; once per process before launches.
 hipError_t init_kernels();
+// Parts of launch_frame and init_kernels for direct frames (direct.hip).
+void launch_front(const BatchParams& Q, FrameParams* jobs, const FrameParams* job0, const DeviceBuffers& B,
+                  hipStream_t s);
+void launch_tile(const BatchParams& Q, const FrameParams* jobs, const DeviceBuffers& B, hipStream_t s);
+hipError_t init_direct_kernels();
 
 // Device scratch of the allocation-free frame (edxr_render_mesh_noalloc): a
 // file-scope __device__ array in pipeline.hip, one copy per device, held until
