@@ -50,6 +50,9 @@ namespace edxr {
 
 namespace {
 constexpr uint32_t kSetupSlots = 4;  // triangle slots per k_setup thread
+constexpr uint32_t kShadeThreads = 512;
+constexpr uint32_t kShadeListTiles = 8192;  // k_shade walks the work list beyond these tiles, with
+constexpr uint32_t kShadeGroups = 16;       // this many workgroups per CU (batch 416 us; 4 per CU 428)
 static_assert(kJobAlign % (kBlock * kSetupSlots) == 0, "a vertex/setup block must not span two jobs");
 }  // namespace
 
@@ -1365,15 +1368,11 @@ __global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, c
     }
 }
 
-// Deferred shading, one pixel per thread and two 512-thread workgroups per
-// tile (16 rows each; smaller workgroups than one per tile schedule better and
-// cost less where the tile is empty): the
-// winner is the minimum (depth, order) key over the tile's segments (the
-// sequential d <= D test is an associative minimum), then perspective-correct
-// interpolation, the pixel shader and one write of colour, depth and
-// triangle ID (Core/Renderer.cpp:272-350).  Empty tiles of single-sample
-// batches are cleared by k_raster.
-
+// Deferred shading, one pixel per thread: the winner is the minimum (depth,
+// order) key over the tile's segments (the sequential d <= D test is an
+// associative minimum), then perspective-correct interpolation, the pixel
+// shader and one write of colour, depth and triangle ID
+// (Core/Renderer.cpp:272-350).
 namespace {
 // Minimum key of sample s over the tile's segment images (S samples per image).
 __device__ __forceinline__ uint64_t tile_key(const uint64_t* g, uint32_t nseg, uint32_t S, uint32_t s) {
@@ -1395,16 +1394,78 @@ __device__ __forceinline__ uint64_t tile_key(const uint64_t* g, uint32_t nseg, u
 }
 }  // namespace
 
+// One pixel (number pix of the tile) of a single-sample frame's nonempty tile.
 template <bool kTex>
-__device__ __forceinline__ void shade_body(const BatchParams& Q, const FrameParams* __restrict__ jobs,
+__device__ __forceinline__ void shade_pixel_of(const FrameParams& P, const DeviceBuffers& B, uint32_t gtile, uint32_t n,
+                                               uint32_t pix) {
+    constexpr uint32_t kPix = kTileSize * kTileSize;
+    const uint32_t tile = gtile - P.tile_base;
+    const int x = (int)(tile % P.tiles_x) * kTileSize + (int)(pix & 31u);
+    const int y = (int)(tile / P.tiles_x) * kTileSize + (int)(pix >> 5);
+    if (x >= (int)P.width || y >= (int)P.height) return;
+    const uint32_t tileItem = B.tile_item[gtile];
+    const uint32_t nseg = tile_segments(n, tileItem >> kImageBits);
+    const uint64_t* g = B.partials + (size_t)(tileItem & kImageMask) * kPix;
+    // A single-segment tile's image holds 32-bit low words (k_raster).
+    uint32_t low;
+    if (nseg == 1) {
+        low = reinterpret_cast<const uint32_t*>(g)[pix];
+    } else {
+        const uint64_t key = tile_key(g + pix, nseg, 1, 0);
+        low = key == bg_key() ? 0xFFFFFFFFu : (uint32_t)key;
+    }
+    shade_winner<kTex>(P, B, x, y, P.pix_base + (size_t)(P.height - 1 - y) * P.width + x, low,
+                       n >= kShadeRecomputeRefs);
+}
+
+// Single-sample frames of up to kShadeListTiles tiles: two workgroups per tile,
+// 16 rows each (smaller workgroups than one per tile schedule better and cost
+// less where the tile is empty, cleared by k_raster).
+template <bool kTex>
+__device__ __forceinline__ void shade_tiles(const BatchParams& Q, const FrameParams* __restrict__ jobs,
+                                            const DeviceBuffers& B) {
+    if (B.counters[kCntOverflow] & kOvNoLists) return;
+    const uint32_t gtile = blockIdx.x >> 1;
+    const uint32_t n = B.tile_start[gtile + 1] - B.tile_start[gtile];
+    if (n == 0) return;
+    shade_pixel_of<kTex>(jobs[job_of(Q, Q.tile_job, gtile)], B, gtile, n,
+                         threadIdx.x + (blockIdx.x & 1u) * kShadeThreads);
+}
+
+// More tiles (batches): the grid's waves take the 16 row pairs of every tile of
+// the work list in turn (a tile's item of segment 0 stands for it), so that no
+// wave is started for an empty tile.  Of the 1.9M waves of two workgroups per
+// tile for 256 jobs three quarters only found their tile empty: 577 us, so 416;
+// 64 views 126 and 81 us.  Where most tiles are covered the list is one load
+// more per tile: 2M sphere grid at 1080p 17 and 20 us, 10M heightfield at 4K 77
+// and 79 us.
+template <bool kTex>
+__device__ __forceinline__ void shade_list(const BatchParams& Q, const FrameParams* __restrict__ jobs,
                                            const DeviceBuffers& B) {
+    constexpr uint32_t kPairs = kTileSize * kTileSize / kWave;
+    if (B.counters[kCntOverflow] & kOvNoLists) return;
+    const uint32_t waves = gridDim.x * (kShadeThreads / kWave);
+    const uint32_t units = B.counters[kCntWorkItems] * kPairs;
+    for (uint32_t u = __builtin_amdgcn_readfirstlane(blockIdx.x * (kShadeThreads / kWave) + threadIdx.x / kWave);
+         u < units; u += waves) {
+        const uint32_t item = __builtin_amdgcn_readfirstlane(B.work[u / kPairs]);
+        if ((item >> kTileBits) & ((1u << kSegIndexBits) - 1)) continue;  // a further segment
+        const uint32_t gtile = item & (kMaxBatchTiles - 1);
+        const uint32_t n = B.tile_start[gtile + 1] - B.tile_start[gtile];
+        shade_pixel_of<kTex>(jobs[job_of(Q, Q.tile_job, gtile)], B, gtile, n, (u % kPairs) * kWave + __lane_id());
+    }
+}
+
+// Multisampled frames: two workgroups per tile, 16 rows each.
+template <bool kTex>
+__device__ __forceinline__ void shade_samples(const BatchParams& Q, const FrameParams* __restrict__ jobs,
+                                              const DeviceBuffers& B) {
     constexpr uint32_t kPix = kTileSize * kTileSize;
     if (B.counters[kCntOverflow] & kOvNoLists) return;
     const uint32_t gtile = blockIdx.x >> 1;
-    const uint32_t pix = threadIdx.x + (blockIdx.x & 1u) * 512u;  // pixel of the tile
+    const uint32_t pix = threadIdx.x + (blockIdx.x & 1u) * kShadeThreads;  // pixel of the tile
     const uint32_t start = B.tile_start[gtile];
     const uint32_t n = B.tile_start[gtile + 1] - start;
-    if (n == 0 && Q.max_samples == 1) return;  // an empty tile, cleared by k_raster
     const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];
     const uint32_t tile = gtile - P.tile_base;
     const int x = (int)(tile % P.tiles_x) * kTileSize + (int)(pix & 31u);
@@ -1414,14 +1475,6 @@ __device__ __forceinline__ void shade_body(const BatchParams& Q, const FramePara
     const uint32_t nseg = tile_segments(n, tileItem >> kImageBits), S = P.samples;
     const uint64_t* g = B.partials + (size_t)(tileItem & kImageMask) * S * kPix + pix;
     const size_t o = P.pix_base + (size_t)(P.height - 1 - y) * P.width + x;
-    if (S == 1) {
-        // A single-segment tile's image holds 32-bit low words (k_raster).
-        const uint64_t key = !n ? bg_key()
-                             : nseg == 1 ? (uint64_t)reinterpret_cast<const uint32_t*>(g - pix)[pix] | 0xBF80000000000000ull
-                                         : tile_key(g, nseg, 1, 0);
-        shade_winner<kTex>(P, B, x, y, o, key == bg_key() ? 0xFFFFFFFFu : (uint32_t)key, n >= kShadeRecomputeRefs);
-        return;
-    }
     // Multisampling: per-sample winners and depths (the sequential LEQUAL test
     // per sample, Core/FrameBuffer.cpp:54-68); a winner is shaded once at the
     // pixel centre (Core/Rasterizer.h:270-285, Core/Renderer.cpp:305-350); the
@@ -1471,15 +1524,24 @@ __device__ __forceinline__ void shade_body(const BatchParams& Q, const FramePara
 }
 
 // Untextured launches are held to 64 VGPRs, so that eight waves per SIMD are
-// resident (two of them spill to scratch outside the pixel's gathers); the
-// texture samplers need more.
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_shade(
-    BatchParams Q, const FrameParams* __restrict__ jobs, DeviceBuffers B) {
-    shade_body<false>(Q, jobs, B);
+// resident; the texture samplers need more.
+enum ShadeMode { kShadeTiles, kShadeList, kShadeSamples };
+template <bool kTex, ShadeMode kMode>
+__device__ __forceinline__ void shade_any_mode(const BatchParams& Q, const FrameParams* __restrict__ jobs,
+                                               const DeviceBuffers& B) {
+    if (kMode == kShadeTiles) shade_tiles<kTex>(Q, jobs, B);
+    else if (kMode == kShadeList) shade_list<kTex>(Q, jobs, B);
+    else shade_samples<kTex>(Q, jobs, B);
 }
-__global__ __launch_bounds__(512) void k_shade_tex(BatchParams Q, const FrameParams* __restrict__ jobs,
-                                                   DeviceBuffers B) {
-    shade_body<true>(Q, jobs, B);
+template <ShadeMode kMode>
+__global__ __launch_bounds__(kShadeThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_shade(
+    BatchParams Q, const FrameParams* __restrict__ jobs, DeviceBuffers B) {
+    shade_any_mode<false, kMode>(Q, jobs, B);
+}
+template <ShadeMode kMode>
+__global__ __launch_bounds__(kShadeThreads) void k_shade_tex(BatchParams Q, const FrameParams* __restrict__ jobs,
+                                                             DeviceBuffers B) {
+    shade_any_mode<true, kMode>(Q, jobs, B);
 }
 
 // ---------------------------------------------------------------------------
@@ -1623,8 +1685,15 @@ hipError_t launch_frame(const BatchParams& Q, FrameParams* jobs, const FramePara
     mark(4);
     if (Q.max_samples > 1) hipLaunchKernelGGL((k_raster<true>), dim3(B.raster_grid), dim3(kBlock), 0, s, Q, jobs, B);
     else hipLaunchKernelGGL((k_raster<false>), dim3(B.raster_grid), dim3(kBlock), 0, s, Q, jobs, B);
-    if (Q.any_textured) hipLaunchKernelGGL(k_shade_tex, dim3(2 * Q.total_tiles), dim3(512), 0, s, Q, jobs, B);
-    else hipLaunchKernelGGL(k_shade, dim3(2 * Q.total_tiles), dim3(512), 0, s, Q, jobs, B);
+    const dim3 shadeThreads(kShadeThreads);
+    auto shade = [&](auto plain, auto textured, dim3 grid) {
+        if (Q.any_textured) hipLaunchKernelGGL(textured, grid, shadeThreads, 0, s, Q, jobs, B);
+        else hipLaunchKernelGGL(plain, grid, shadeThreads, 0, s, Q, jobs, B);
+    };
+    if (Q.max_samples > 1) shade(k_shade<kShadeSamples>, k_shade_tex<kShadeSamples>, dim3(2 * Q.total_tiles));
+    else if (Q.total_tiles > kShadeListTiles)
+        shade(k_shade<kShadeList>, k_shade_tex<kShadeList>, dim3(kShadeGroups * B.num_cus));
+    else shade(k_shade<kShadeTiles>, k_shade_tex<kShadeTiles>, dim3(2 * Q.total_tiles));
     mark(5);
     return hipGetLastError();
 }
