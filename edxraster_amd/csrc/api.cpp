@@ -141,12 +141,10 @@ struct JobInput {
     int32_t shader, hierarchical;
 };
 
-// A batch laid out for launch_frame: job table, batch sizes, block -> job
-// tables (vertex blocks | setup blocks | chunks | tiles) and buffer sizes.
+// A batch laid out for launch_frame: job table, batch sizes and buffer sizes.
 struct Plan {
     std::vector<FrameParams> jobs;
     BatchParams Q{};
-    std::vector<uint32_t> tables;
     uint64_t countEntries = 0, groupEntries = 0, pixels = 0;
 };
 
@@ -197,7 +195,6 @@ struct edxr_ctx {
     DevBuf<FrameParams> jobsDev;
     DevBuf<uint32_t> jobTables;
     HostBuf<FrameParams> jobsHost;
-    HostBuf<uint32_t> tablesHost;
     // batch outputs
     DevBuf<uint32_t> bcolor, bids;
     DevBuf<float> bdepth;
@@ -387,12 +384,11 @@ FrameParams job_params(const JobInput& in, uint32_t tilesX, uint32_t tilesY) {
 }
 
 // Places the jobs in the batch arrays.  Vertex and triangle slots start on
-// kJobAlign boundaries so each block of k_vertex / k_setup belongs to one job;
-// the block -> job tables have one entry per kJobTableBlock slots.
+// kJobAlign boundaries so each block of k_vertex / k_setup belongs to one job.
 int build_plan(edxr_ctx* c, const std::vector<JobInput>& in, Plan& pl) {
     const bool single = in.size() == 1;
     pl.jobs.clear();
-    pl.tables.clear();
+    pl.jobs.reserve(in.size());
     uint64_t vert = 0, slot = 0, tile = 0, chunk = 0;
     pl.countEntries = pl.groupEntries = pl.pixels = 0;
     BatchParams& Q = pl.Q;
@@ -434,25 +430,6 @@ int build_plan(edxr_ctx* c, const std::vector<JobInput>& in, Plan& pl) {
     Q.total_chunks = (uint32_t)chunk;
     Q.vert_blocks = (uint32_t)((vert + kJobTableBlock - 1) / kJobTableBlock);
     Q.slot_blocks = (uint32_t)((slot + kJobTableBlock - 1) / kJobTableBlock);
-    if (!single) {
-        pl.tables.resize((size_t)Q.vert_blocks + Q.slot_blocks + Q.total_chunks + Q.total_tiles);
-        uint32_t* vb = pl.tables.data();
-        uint32_t* sb = vb + Q.vert_blocks;
-        uint32_t* cj = sb + Q.slot_blocks;
-        uint32_t* tj = cj + Q.total_chunks;
-        // Padding blocks up to the next job's base belong to the job before it.
-        for (uint32_t k = 0; k < Q.num_jobs; k++) {
-            const FrameParams& P = pl.jobs[k];
-            const uint32_t vEnd = k + 1 < Q.num_jobs ? pl.jobs[k + 1].vert_base : Q.total_verts;
-            const uint32_t sEnd = k + 1 < Q.num_jobs ? pl.jobs[k + 1].slot_base : Q.total_slots;
-            for (uint32_t b = P.vert_base / kJobTableBlock; b < (vEnd + kJobTableBlock - 1) / kJobTableBlock; b++)
-                vb[b] = k;
-            for (uint32_t b = P.slot_base / kJobTableBlock; b < (sEnd + kJobTableBlock - 1) / kJobTableBlock; b++)
-                sb[b] = k;
-            for (uint32_t i = 0; i < P.num_chunks; i++) cj[P.chunk_base + i] = k;
-            for (uint32_t i = 0; i < P.num_tiles; i++) tj[P.tile_base + i] = k;
-        }
-    }
     return EDXR_OK;
 }
 
@@ -555,14 +532,9 @@ int run_plan(edxr_ctx* c, Plan& pl, uint32_t* color, float* depth, uint32_t* ids
                                 hipMemcpyHostToDevice, c->stream)) != hipSuccess)
             return c->hip_fail(e, "hipMemcpyAsync(jobs)");
     }
-    if (!pl.tables.empty()) {
-        if ((e = c->jobTables.ensure(pl.tables.size())) != hipSuccess ||
-            (e = c->tablesHost.ensure(pl.tables.size())) != hipSuccess)
+    if (!single) {
+        if ((e = c->jobTables.ensure((size_t)Q.vert_blocks + Q.slot_blocks + Q.total_chunks + Q.total_tiles)) != hipSuccess)
             return c->hip_fail(e, "hipMalloc(job tables)");
-        memcpy(c->tablesHost.p, pl.tables.data(), 4 * pl.tables.size());
-        if ((e = hipMemcpyAsync(c->jobTables.p, c->tablesHost.p, 4 * pl.tables.size(), hipMemcpyHostToDevice,
-                                c->stream)) != hipSuccess)
-            return c->hip_fail(e, "hipMemcpyAsync(job tables)");
         Q.vblock_job = c->jobTables.p;
         Q.sblock_job = Q.vblock_job + Q.vert_blocks;
         Q.chunk_job = Q.sblock_job + Q.slot_blocks;
@@ -921,7 +893,6 @@ void edxr_destroy(edxr_ctx* c) {
     c->sverts.release();
     c->jobsDev.release();
     c->jobsHost.release();
-    c->tablesHost.release();
     if (c->hostCounters) (void)hipHostFree(c->hostCounters);
     for (auto& ev : c->events)
         if (ev) (void)hipEventDestroy(ev);
@@ -1369,9 +1340,6 @@ int edxr_render_batch(edxr_ctx* c, const edxr_job* jobs, uint32_t n) {
     if ((r = run_plan(c, pl, c->bcolor.p, c->bdepth.p, c->bids.p, c->floatColor ? c->bcolorF.p : nullptr)) !=
         EDXR_OK)
         return r;
-    c->lastPlan = pl;
-    c->lastPlanValid = true;
-    c->lastFloat = c->floatColor != 0;
     c->batchPix.resize(n + 1);
     c->batchW.resize(n);
     c->batchH.resize(n);
@@ -1381,6 +1349,9 @@ int edxr_render_batch(edxr_ctx* c, const edxr_job* jobs, uint32_t n) {
         c->batchH[k] = pl.jobs[k].height;
     }
     c->batchPix[n] = pl.pixels;
+    c->lastPlan = std::move(pl);
+    c->lastPlanValid = true;
+    c->lastFloat = c->floatColor != 0;
     c->batchRendered = true;
     return EDXR_OK;
 }

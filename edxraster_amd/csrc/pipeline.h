@@ -126,7 +126,9 @@ struct FrameParams {
     uint32_t num_tex, tex_filter;
 };
 
-// Batch-wide sizes and the block -> job tables (null for a single job).
+// Batch-wide sizes and the block -> job tables (null for a single job; filled by
+// k_job_tables): one entry per kJobTableBlock vertex or triangle slots, per
+// chunk, per tile.
 struct BatchParams {
     uint32_t num_jobs;
     uint32_t total_slots;    // triangle slots; clipped pieces' records follow
