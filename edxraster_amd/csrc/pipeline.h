@@ -50,7 +50,7 @@ constexpr uint32_t kDirectFewTiles = 8192;
 constexpr uint32_t kDirectHeavy = 48;
 constexpr uint32_t kDirectMaxTiles = 32768;
 constexpr uint32_t kDirectMaxSlots = 1u << 20;  // triangle slots of a direct frame,
-constexpr uint32_t kDirectSlots = 512;          // and per tile on average, at most
+constexpr uint32_t kDirectSlots = 416;          // and per tile on average, at most
 constexpr uint32_t kScanSpinLimit = 1u << 20;  // k_bin_colpass look-back waits (about 30 ms) before giving up
 // Single-sample shading rebuilds a winner's screen values from its shading
 // vertices, instead of gathering them, in tiles of this many references or

@@ -2,7 +2,7 @@
 tile) against the general path over the forms they accept, bit for bit, and
 against the oracle at the limits that send a frame to the general path: a
 tile's references (4,096; 2,048 in the allocation-free frame and beyond 8,192
-tiles) and tile-level triangles (48), 512 triangle slots per tile, 32,768
+tiles) and tile-level triangles (48), 416 triangle slots per tile, 32,768
 tiles.  The general path is taken with a chunk count set by the caller (single
 frames) or with the capacity testing aid (batches)."""
 import numpy as np
@@ -68,8 +68,8 @@ SCENES = {
     "textured": lambda: configs.textured_scene(320, 200, 40),
     "reference_shader": lambda: _shader(configs.heightfield_small(60, 200, 150), 1, 200.0),
     "lambert": lambda: _shader(configs.heightfield_small(60, 2047, 2048), 0, 0.0),
-    "below_slots": lambda: configs.small_sphere(96, 32, 48, 16),     # 1,536 triangles on 3 tiles: 512 a tile
-    "above_slots": lambda: configs.small_sphere(96, 32, 49, 16),
+    "below_slots": lambda: configs.small_sphere(96, 32, 39, 16),     # 1,248 triangles on 3 tiles: 416 a tile
+    "above_slots": lambda: configs.small_sphere(96, 32, 40, 16),
     "tile_4095": lambda: small_in_one_tile(4095), "tile_4096": lambda: small_in_one_tile(4096),
     "tile_4097": lambda: small_in_one_tile(4097),
     "large_47": lambda: large(47), "large_48": lambda: large(48), "large_49": lambda: large(49),
