@@ -281,10 +281,6 @@ int set_size(edxr_ctx* c, uint32_t w, uint32_t h) {
     return EDXR_OK;
 }
 
-// Binning chunks of a job: about trisPerChunk (1024) triangles each so the
-// count/scatter grids fill the GPU, capped so the job's chunk x tile count
-// matrix (allocated in full, touched only inside each chunk's tile box) stays
-// within matrixBytes.
 // Sums of the striped counters of a frame (h: the counters read back).  The
 // clip stage allocates from kAllocStripes regions; a capacity that holds its
 // fullest stripe's demand in every region is that demand times the stripes.
@@ -313,6 +309,16 @@ CounterSums counter_sums(const uint32_t* h) {
     return cs;
 }
 
+// Binning chunks of a job: about trisPerChunk (1024) triangles each so the
+// count/scatter grids fill the GPU, capped so the job's chunk x tile count
+// matrix (allocated in full, touched only inside each chunk's tile box) stays
+// within matrixBytes.  Without a setting, jobs of more than kChunkFewTiles tiles
+// have at most kChunksManyTiles chunks: every chunk's box is a stretch of the
+// matrix there, written, scanned and read, and 2,048 chunks already fill the GPU.
+// At 4K with 4,096 chunks and with 2,048: 10M heightfield 511 and 499 us, 3.1M
+// 280 and 272, 5.8M sphere 283 and 267, 4.1M sphere grid 267 and 257; at 1080p
+// the 4.1M grid takes 182 and 184, and below 2,048 chunks the 2.1M grid at 4K
+// gets slower (232 us with 2,048, 241 with 1,024).
 uint32_t choose_chunks(const edxr_ctx* c, uint32_t T, uint32_t nTiles, bool single,
                        uint64_t matrixBytes = 256ull << 20) {
     if (T == 0) return 0;
@@ -320,8 +326,9 @@ uint32_t choose_chunks(const edxr_ctx* c, uint32_t T, uint32_t nTiles, bool sing
     if (single && c->binChunksSetting)
         return std::max(1u, std::min(std::min(std::min(c->binChunksSetting, kMaxChunks), T), byMatrix));
     const uint32_t tpc = c->trisPerChunk ? c->trisPerChunk : 1024;
+    const uint32_t most = !c->trisPerChunk && nTiles > kChunkFewTiles ? kChunksManyTiles : kMaxChunks;
     const uint32_t C = (T + tpc - 1) / tpc;
-    return std::max(1u, std::min(std::min(C, byMatrix), kMaxChunks));
+    return std::max(1u, std::min(std::min(C, byMatrix), most));
 }
 
 int check_mesh(edxr_ctx* c, const edxr_mesh* m, int32_t shader) {

@@ -59,6 +59,8 @@ constexpr uint32_t kShadeRecomputeRefs = 512;
 constexpr uint32_t kJobAlign = 1024;         // job slot alignment: vertex/setup blocks never span jobs
 constexpr uint32_t kJobTableBlock = 256;     // slots (vertices) per entry of the block -> job tables
 constexpr uint32_t kMaxChunks = 4096;
+constexpr uint32_t kChunkFewTiles = 4096;    // (choose_chunks)
+constexpr uint32_t kChunksManyTiles = 2048;
 // Per-triangle descriptor: bit 31 set = compact small triangle (record in slot
 // t; tile bbox minTX | minTY << 14 | dx << 28 | dy << 29, dx, dy in {0, 1});
 // otherwise (first record << 3) | record count (0..7).

@@ -59,3 +59,22 @@ def test_noalloc_equals_plain_frame(built, size):
     assert r.stats()["clipped"] > 0
     assert_equal_frames(got, plain_frame(r, w), "%dx%d" % size)
     r.close()
+
+
+@pytest.mark.parametrize("size", [(2048, 2048), (65 * 32, 2048)], ids=["4096", "4160"])
+def test_default_chunks_of_many_triangles(built, size):
+    """2.2M triangles: the default number of binning chunks on either side of
+    4,096 tiles, the frame as with every other number."""
+    w = configs.heightfield_small(1050, size[0], size[1], seed=5)
+    r = Renderer(w.width, w.height)
+    w.apply(r)
+    frames = []
+    for chunks in (0, 4096, 700):
+        r.set_bin_chunks(chunks)
+        r.render_mesh(w.mesh)
+        if chunks == 0:
+            assert r.stats()["bin_chunks"] == (2048 if size[0] > 2048 else 2150)
+        frames.append((r.get_back_buffer(), r.read_depth().view(np.uint32), r.read_triangle_ids()))
+    for f in frames[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(f, frames[0]))
+    r.close()
