@@ -422,8 +422,8 @@ __global__ __launch_bounds__(kAdjBlock, 3) void k_adjoint(BatchParams Q, const F
     __syncthreads();  // the places are read: count takes the vertices' slots
     for (uint32_t i = threadIdx.x; i < S.nTri; i += kAdjBlock) {
         const uint32_t e = S.triUsed[i];
-        const uint32_t* idx = P.mesh.idx + 3 * (size_t)S.tri[e];
-        const uint32_t v0 = idx[0], v1 = idx[1], v2 = idx[2];
+        const size_t t = 3 * (size_t)S.tri[e];
+        const uint32_t v0 = at(P.mesh.idx, t), v1 = at(P.mesh.idx, t + 1), v2 = at(P.mesh.idx, t + 2);
         S.count[e] = vertex_slot(S, v0) | vertex_slot(S, v1) << kVertSlotBits | vertex_slot(S, v2) << 2 * kVertSlotBits;
     }
     __syncthreads();

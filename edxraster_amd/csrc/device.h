@@ -19,6 +19,20 @@ constexpr uint32_t kWave = 64;
 constexpr uint32_t kBlock = 256;
 static_assert(kBlock == kJobTableBlock, "block -> job tables are indexed by 256-slot block");
 
+// p in device memory.  A pointer read from memory would be loaded through as a
+// generic one, and such a load also counts against the LDS waits: a kernel that
+// loads ahead and works in LDS then waits for its loads with each LDS result.
+template <class T>
+using GlobalPtr = const __attribute__((address_space(1))) T*;
+template <class T>
+__device__ __forceinline__ GlobalPtr<T> as_global(const T* p) {
+    return (GlobalPtr<T>)p;
+}
+template <class T>
+__device__ __forceinline__ T global_at(const T* p, size_t i) {
+    return as_global(p)[i];
+}
+
 __device__ __forceinline__ float4 xform4(const float* m, float x, float y, float z, float w) {
     float4 r;
     r.x = ((m[0] * x + m[1] * y) + m[2] * z) + m[3] * w;
@@ -56,13 +70,6 @@ __device__ __forceinline__ int2 snap_point(const FrameParams& P, float ax, float
     const float4 A = xform4(P.raster, ax, ay, az, 1.0f);
     if (A.w == 1.0f) return make_int2(snap(A.x), snap(A.y));
     return make_int2(snap(A.x / A.w), snap(A.y / A.w));
-}
-
-// p[i] of device memory (a pointer read from memory would be loaded through as
-// a generic one, which also counts against the LDS waits).
-template <class T>
-__device__ __forceinline__ T global_at(const T* p, size_t i) {
-    return ((const __attribute__((address_space(1))) T*)p)[i];
 }
 
 // RasterTriangle::Setup from snapped vertices (Core/RasterTriangle.h:42-153);
@@ -169,7 +176,7 @@ __device__ __forceinline__ void vertex_slot(const FrameParams& P, uint32_t slot,
     const MeshPtrs& M = P.mesh;
     const uint32_t v = slot - P.vert_base;
     if (v >= P.num_vertices) return;
-    const float px = M.px[v], py = M.py[v], pz = M.pz[v];
+    const float px = global_at(M.px, v), py = global_at(M.py, v), pz = global_at(M.pz, v);
     // DefaultVertexShader::Execute: projectedPos = MVP * (p, 1); the outcode,
     // the homogeneous projection and the snapped raster position are per
     // vertex, so every unclipped triangle's setup reuses them.
@@ -184,15 +191,15 @@ __device__ __forceinline__ void vertex_slot(const FrameParams& P, uint32_t slot,
         o.px = px;
         o.py = py;
         o.pz = pz;
-        o.nx = M.nx[v];
-        o.ny = M.ny[v];
-        o.nz = M.nz[v];
-        o.cr = M.cr ? M.cr[v] : 0.0f;
-        o.cg = M.cg ? M.cg[v] : 0.0f;
-        o.cb = M.cb ? M.cb[v] : 0.0f;
+        o.nx = global_at(M.nx, v);
+        o.ny = global_at(M.ny, v);
+        o.nz = global_at(M.nz, v);
+        o.cr = M.cr ? global_at(M.cr, v) : 0.0f;
+        o.cg = M.cg ? global_at(M.cg, v) : 0.0f;
+        o.cb = M.cb ? global_at(M.cb, v) : 0.0f;
         o.inv_w = 1.0f / c.w;
-        o.u = M.tu ? M.tu[v] : 0.0f;
-        o.v = M.tv ? M.tv[v] : 0.0f;
+        o.u = M.tu ? global_at(M.tu, v) : 0.0f;
+        o.v = M.tv ? global_at(M.tv, v) : 0.0f;
         verts[slot] = o;
     }
     sverts[slot] = sv;
@@ -204,7 +211,9 @@ namespace {
 // tile bbox spans at most 2x2 tiles, binning lists it in every bbox tile with
 // no corner test (Core/Renderer.cpp:168-180), so the bbox alone (packed here,
 // in the job's tile coordinates) enumerates its references; otherwise
-// (t << 3) | 1.
+// (t << 3) | 1.  Only a triangle shorter than kCompactExtent is compact (others
+// of so small a clamped bbox reach far off the screen): the raster kernels
+// take products of a compact triangle's differences in 24 bits.
 __device__ __forceinline__ uint32_t compact_desc(const FrameParams& P, const RasterRec& r, uint32_t t) {
     const int Shift = kTileLog2 + 4;
     const int minTX = max(0, min(r.x0, min(r.x1, r.x2)) >> Shift);
@@ -213,9 +222,11 @@ __device__ __forceinline__ uint32_t compact_desc(const FrameParams& P, const Ras
     const int maxTY = min((int)P.tiles_y - 1, max(r.y0, max(r.y1, r.y2)) >> Shift);
     const int dx = maxTX - minTX, dy = maxTY - minTY;
     if (dx < 0 || dy < 0 || dx > 1 || dy > 1) return (t << 3) | 1u;
+    const uint32_t ex = (uint32_t)max(r.x0, max(r.x1, r.x2)) - (uint32_t)min(r.x0, min(r.x1, r.x2));
+    const uint32_t ey = (uint32_t)max(r.y0, max(r.y1, r.y2)) - (uint32_t)min(r.y0, min(r.y1, r.y2));
+    if (max(ex, ey) >= kCompactExtent) return (t << 3) | 1u;
     // a pixel bounding box of kHeavyPixels or more: a whole wave's work in the raster
-    const int bw = (max(r.x0, max(r.x1, r.x2)) - min(r.x0, min(r.x1, r.x2))) >> 4;
-    const int bh = (max(r.y0, max(r.y1, r.y2)) - min(r.y0, min(r.y1, r.y2))) >> 4;
+    const int bw = (int)(ex >> 4), bh = (int)(ey >> 4);
     const uint32_t heavy = bw * bh >= (int)kHeavyPixels ? kDescHeavy : 0u;
     return kDescCompact | heavy | (uint32_t)minTX | ((uint32_t)minTY << 14) | ((uint32_t)dx << 28) |
            ((uint32_t)dy << 29);
@@ -443,7 +454,17 @@ __device__ __forceinline__ void load_rtri(const RasterRec& r, RTri& t) {
     t.order = r.order;
 }
 
-// Record of an unclipped triangle in slot r from its vertices' screen values
+// a * b of 24-bit values in 32 bits, cheaper than a 32-bit product (k_raster of
+// the 10M heightfield at 4K, bound by its vector instructions: 121 us with 32-bit
+// products, 119 with these).
+__device__ __forceinline__ int mul24(int a, int b) { return __mul24(a, b); }
+template <bool kShort>
+__device__ __forceinline__ int mul(int a, int b) { return kShort ? __mul24(a, b) : a * b; }
+// pixel_bias of a compact triangle's edge, whose B and C fit 16 bits: B < 0, or
+// B == 0 and C < 0.
+__device__ __forceinline__ int compact_bias(int B, int C) { return ((int)((uint32_t)B << 16) + C) >> 31; }
+
+// Record of a compact triangle in slot r from its vertices' screen values
 // (the values k_setup used); corner codes are not needed below tile level.
 __device__ __forceinline__ void screen_rtri_from(const ScreenVert& s0, const ScreenVert& s1, const ScreenVert& s2,
                                                  uint32_t r, RTri& t) {
@@ -451,26 +472,32 @@ __device__ __forceinline__ void screen_rtri_from(const ScreenVert& s0, const Scr
     t.B0 = t.y0 - t.y1; t.C0 = t.x1 - t.x0;
     t.B1 = t.y1 - t.y2; t.C1 = t.x2 - t.x1;
     t.B2 = t.y2 - t.y0; t.C2 = t.x0 - t.x2;
-    t.pb0 = pixel_bias(t.x0, t.y0, t.x1, t.y1);
-    t.pb1 = pixel_bias(t.x1, t.y1, t.x2, t.y2);
-    t.pb2 = pixel_bias(t.x2, t.y2, t.x0, t.y0);
-    t.inv_det = 1.0f / (float)(t.C2 * t.B1 - t.C1 * t.B2);
+    t.pb0 = compact_bias(t.B0, t.C0);
+    t.pb1 = compact_bias(t.B1, t.C1);
+    t.pb2 = compact_bias(t.B2, t.C2);
+    t.inv_det = 1.0f / (float)(mul24(t.C2, t.B1) - mul24(t.C1, t.B2));
     t.z0 = s0.z; t.z1 = s1.z; t.z2 = s2.z;
     t.info = 0;
     t.order = make_order(r, 0, false);
 }
 __device__ __forceinline__ void screen_rtri(const FrameParams& P, const DeviceBuffers& B, uint32_t r, RTri& t) {
-    const uint32_t* idx = P.mesh.idx + 3 * (size_t)(r - P.slot_base);
+    const GlobalPtr<uint32_t> idx = as_global(P.mesh.idx) + 3 * (size_t)(r - P.slot_base);
     screen_rtri_from(B.sverts[P.vert_base + idx[0]], B.sverts[P.vert_base + idx[1]], B.sverts[P.vert_base + idx[2]],
                      r, t);
 }
+// Whether differences of the triangle's coordinates and of pixels fit 24 bits
+// (any triangle's do whose raster matrix maps to a picture of the usual size).
+__device__ __forceinline__ bool fits24(const RTri& t) {
+    auto out = [](int v) { return (uint32_t)v + (1u << 22) >= (2u << 22); };
+    return !(out(t.x0) | out(t.y0) | out(t.x1) | out(t.y1) | out(t.x2) | out(t.y2));
+}
 
 // A reference's index-buffer entries when it is a compact unclipped triangle
-// (otherwise the job's first entries, a valid address whose value is unused).
-__device__ __forceinline__ uint3 ref_indices(const FrameParams& P, uint32_t total_slots, uint32_t pay) {
-    const uint32_t rid = pay & kRecordMask;
-    const bool compact = !(pay >> 31) && rid < total_slots && rid >= P.slot_base;
-    const uint32_t* idx = P.mesh.idx + (compact ? 3 * (size_t)(rid - P.slot_base) : 0);
+// (otherwise another triangle's of the job, a valid address whose value is
+// unused).
+__device__ __forceinline__ uint3 ref_indices(const FrameParams& P, uint32_t pay) {
+    const uint32_t k = min((pay & kRecordMask) - P.slot_base, P.num_triangles - 1u);
+    const GlobalPtr<uint32_t> idx = as_global(P.mesh.idx) + 3 * (size_t)k;
     return make_uint3(idx[0], idx[1], idx[2]);
 }
 
@@ -499,11 +526,22 @@ constexpr int kKeyStride = kMS ? kTileSize : kTileSize + 1;
 template <bool kMS>
 constexpr uint32_t kKeyPlane = kTileSize * kKeyStride<kMS>;
 
-// Samples of one raster pass: MSAA level, first sample and count; sample
-// k's keys live in plane k (kKeyPlane<true> keys apart).
+// Samples of one raster pass: their count, and their offsets, a byte each (x in
+// the low four bits, y in the high); sample k's keys live in plane k
+// (kKeyPlane<true> keys apart).
 struct SamplePass {
-    uint32_t level, base, n;
+    uint32_t n, offsets;
 };
+// Loaded once per pass: a load per sample of every pixel waited with each for
+// the LDS atomics before it (one counter).
+__device__ __forceinline__ SamplePass sample_pass(uint32_t level, uint32_t base, uint32_t n) {
+    uint32_t offsets = 0;
+    for (uint32_t k = 0; k < n; k++) {
+        const int2 o = c_sample_offsets[level][base + k];
+        offsets |= (((uint32_t)o.x & 15u) | ((uint32_t)o.y & 15u) << 4) << (8 * k);
+    }
+    return SamplePass{n, (uint32_t)__builtin_amdgcn_readfirstlane(offsets)};
+}
 
 // Depth test of one pixel from its edge values e0..e2 (coverage when
 // useEdges, Core/Rasterizer.h:162), then the (depth, order) key update; klo is
@@ -514,7 +552,8 @@ struct SamplePass {
 // it holds in wrapping int32 as well.  With multisampling each sample of the
 // pass is tested at centre + offset (Core/Rasterizer.h:243-266):
 // e + ox B + oy C, wrapping as the reference.
-template <bool kMS>
+// kShort: differences of the triangle's coordinates fit 24 bits.
+template <bool kMS, bool kShort>
 __device__ __forceinline__ void pixel_key(const RTri& t, int e0, int e1, int e2, uint32_t klo, bool useEdges,
                                           uint64_t* slot, const SamplePass& sp) {
     const int n0 = e1 - t.pb1, n1 = e2 - t.pb2;
@@ -531,15 +570,15 @@ __device__ __forceinline__ void pixel_key(const RTri& t, int e0, int e1, int e2,
         return;
     }
     for (uint32_t k = 0; k < sp.n; k++) {
-        const int2 o = c_sample_offsets[sp.level][sp.base + k];
+        const int ox = (int)(sp.offsets << (28 - 8 * k)) >> 28, oy = (int)(sp.offsets << (24 - 8 * k)) >> 28;
+        const int m0 = n0 + mul<kShort>(ox, t.B1) + mul<kShort>(oy, t.C1);
+        const int m1 = n1 + mul<kShort>(ox, t.B2) + mul<kShort>(oy, t.C2);
         if (useEdges) {
-            const int s0 = e0 + o.x * t.B0 + o.y * t.C0;
-            const int s1 = e1 + o.x * t.B1 + o.y * t.C1;
-            const int s2 = e2 + o.x * t.B2 + o.y * t.C2;
-            if ((s0 | s1 | s2) < 0) continue;
+            const int s0 = e0 + mul<kShort>(ox, t.B0) + mul<kShort>(oy, t.C0);
+            if ((s0 | (m0 + t.pb1) | (m1 + t.pb2)) < 0) continue;
         }
-        const float l0 = (float)(n0 + o.x * t.B1 + o.y * t.C1) * t.inv_det;
-        const float l1 = (float)(n1 + o.x * t.B2 + o.y * t.C2) * t.inv_det;
+        const float l0 = (float)m0 * t.inv_det;
+        const float l1 = (float)m1 * t.inv_det;
         const float l2 = 1.0f - l0 - l1;
         const float d = l0 * t.z0 + l1 * t.z1 + l2 * t.z2;
         if (!(d <= 1.0f)) continue;
@@ -554,28 +593,28 @@ __device__ __forceinline__ void pixel_key(const RTri& t, int e0, int e1, int e2,
 // 16 B and 16 C to the other pixels, which is
 // exact in wrapping int32 arithmetic (the reference steps the same way,
 // Core/Rasterizer.h:190-198).
-template <bool kMS>
+template <bool kMS, bool kShort>
 __device__ __forceinline__ void quad_depth(const RTri& t, int qx, int qy, bool useEdges, int tminX, int tminY,
                                            uint64_t* keys, int maxX, int maxY, const SamplePass& sp) {
     const int px = qx * 16 + 8, py = qy * 16 + 8;
-    const int e0 = t.B0 * (px - t.x0) + t.C0 * (py - t.y0) + t.pb0;
-    const int e1 = t.B1 * (px - t.x1) + t.C1 * (py - t.y1) + t.pb1;
-    const int e2 = t.B2 * (px - t.x2) + t.C2 * (py - t.y2) + t.pb2;
+    const int e0 = mul<kShort>(t.B0, px - t.x0) + mul<kShort>(t.C0, py - t.y0) + t.pb0;
+    const int e1 = mul<kShort>(t.B1, px - t.x1) + mul<kShort>(t.C1, py - t.y1) + t.pb1;
+    const int e2 = mul<kShort>(t.B2, px - t.x2) + mul<kShort>(t.C2, py - t.y2) + t.pb2;
     const int sB0 = t.B0 * 16, sB1 = t.B1 * 16, sB2 = t.B2 * 16;
     const int sC0 = t.C0 * 16, sC1 = t.C1 * 16, sC2 = t.C2 * 16;
     const uint32_t klo = 0xFFFFFFFEu - t.order;
     uint64_t* row = &keys[(qy - tminY) * kKeyStride<kMS> + (qx - tminX)];
     const bool right = qx + 1 <= maxX, down = qy + 1 <= maxY;
-    pixel_key<kMS>(t, e0, e1, e2, klo, useEdges, row, sp);
-    if (right) pixel_key<kMS>(t, e0 + sB0, e1 + sB1, e2 + sB2, klo, useEdges, row + 1, sp);
-    if (down) pixel_key<kMS>(t, e0 + sC0, e1 + sC1, e2 + sC2, klo, useEdges, row + kKeyStride<kMS>, sp);
+    pixel_key<kMS, kShort>(t, e0, e1, e2, klo, useEdges, row, sp);
+    if (right) pixel_key<kMS, kShort>(t, e0 + sB0, e1 + sB1, e2 + sB2, klo, useEdges, row + 1, sp);
+    if (down) pixel_key<kMS, kShort>(t, e0 + sC0, e1 + sC1, e2 + sC2, klo, useEdges, row + kKeyStride<kMS>, sp);
     if (right && down)
-        pixel_key<kMS>(t, e0 + sB0 + sC0, e1 + sB1 + sC1, e2 + sB2 + sC2, klo, useEdges, row + kKeyStride<kMS> + 1, sp);
+        pixel_key<kMS, kShort>(t, e0 + sB0 + sC0, e1 + sB1 + sC1, e2 + sB2 + sC2, klo, useEdges, row + kKeyStride<kMS> + 1, sp);
 }
-template <bool kMS>
+template <bool kMS, bool kShort>
 __device__ __forceinline__ void quad_depth(const RTri& t, int qx, int qy, bool useEdges, int tminX, int tminY,
                                            uint64_t* keys, const SamplePass& sp) {
-    quad_depth<kMS>(t, qx, qy, useEdges, tminX, tminY, keys, qx + 1, qy + 1, sp);
+    quad_depth<kMS, kShort>(t, qx, qy, useEdges, tminX, tminY, keys, qx + 1, qy + 1, sp);
 }
 
 __device__ __forceinline__ float pow_decl(float x, int n, float s) {
@@ -662,6 +701,7 @@ __device__ __forceinline__ int tex_wrap(int i, int n) {
     i %= n;
     return i < 0 ? i + n : i;
 }
+typedef float Texel __attribute__((ext_vector_type(4)));
 // A mip level: its first texel and sides.
 struct TexLevel {
     uint32_t off;
@@ -679,8 +719,8 @@ __device__ __forceinline__ float3 tex_bilinear(const FrameParams& P, const TexLe
     const uint32_t i0 = (uint32_t)tex_wrap(tex_index(x0), L.w), j0 = (uint32_t)tex_wrap(tex_index(y0), L.h);
     const uint32_t i1 = i0 + 1 == (uint32_t)L.w ? 0u : i0 + 1, j1 = j0 + 1 == (uint32_t)L.h ? 0u : j0 + 1;
     const uint32_t r0 = L.off + j0 * (uint32_t)L.w, r1 = L.off + j1 * (uint32_t)L.w;
-    const float4 c00 = P.texels[r0 + i0], c10 = P.texels[r0 + i1];
-    const float4 c01 = P.texels[r1 + i0], c11 = P.texels[r1 + i1];
+    const GlobalPtr<Texel> texels = as_global((const Texel*)P.texels);
+    const Texel c00 = texels[r0 + i0], c10 = texels[r0 + i1], c01 = texels[r1 + i0], c11 = texels[r1 + i1];
     const float gx = 1.0f - fx, gy = 1.0f - fy;
     return make_float3(gy * (gx * c00.x + fx * c10.x) + fy * (gx * c01.x + fx * c11.x),
                        gy * (gx * c00.y + fx * c10.y) + fy * (gx * c01.y + fx * c11.y),
@@ -728,7 +768,7 @@ __device__ __forceinline__ float3 tex_sample(const FrameParams& P, const TexDesc
     if (P.tex_filter == kFilterNearest) {
         const uint32_t i = (uint32_t)tex_wrap(tex_index(floorf(u * (float)w)), w);
         const uint32_t j = (uint32_t)tex_wrap(tex_index(floorf(v * (float)h)), h);
-        const float4 c = P.texels[d.offset + j * (uint32_t)w + i];
+        const Texel c = as_global((const Texel*)P.texels)[d.offset + j * (uint32_t)w + i];
         return make_float3(c.x, c.y, c.z);
     }
     if (P.tex_filter == kFilterLinear) return tex_bilinear(P, TexLevel{d.offset, w, h}, u, v);
@@ -815,7 +855,7 @@ __device__ __forceinline__ float3 shade_any(const FrameParams& P, const RTri& t,
                                             float l0, float l1, const ShadeVert& v0, const ShadeVert& v1,
                                             const ShadeVert& v2) {
     if (kTex && P.shader == kTexturedLambert)
-        return shade_textured(P, t, x, y, l0, l1, v0, v1, v2, P.mesh.tex[(order >> 4) - P.slot_base]);
+        return shade_textured(P, t, x, y, l0, l1, v0, v1, v2, global_at(P.mesh.tex, (order >> 4) - P.slot_base));
     return shade_pixel(P, l0, l1, v0, v1, v2);
 }
 
@@ -840,7 +880,7 @@ __device__ __forceinline__ void raster_large_wave(const FrameParams& P, const RT
         // TrivialAcceptTriangle over the tile (Core/Rasterizer.h:310-353).
         for (int q = 0; q < 4; q++) {
             const int qx = tminX + 16 * (q & 1) + lx, qy = tminY + 16 * (q >> 1) + ly;
-            if (qx <= tmaxX - 1 && qy <= tmaxY - 1) quad_depth<kMS>(t, qx, qy, false, tminX, tminY, keys, sp);
+            if (qx <= tmaxX - 1 && qy <= tmaxY - 1) quad_depth<kMS, false>(t, qx, qy, false, tminX, tminY, keys, sp);
         }
     } else {
         // CoarseRasterize (Core/Rasterizer.h:32-111): stepped corner tests per 16x16 quadrant.
@@ -884,14 +924,14 @@ __device__ __forceinline__ void raster_large_wave(const FrameParams& P, const RT
             const int qx = tminX + 16 * (q & 1) + lx, qy = tminY + 16 * (q >> 1) + ly;
             if (acc) {
                 if (qx >= bminX && qx <= bmaxX - 1 && qy >= bminY && qy <= bmaxY - 1)
-                    quad_depth<kMS>(t, qx, qy, false, tminX, tminY, keys, sp);
+                    quad_depth<kMS, false>(t, qx, qy, false, tminX, tminY, keys, sp);
             } else {
                 int minX = max(bminX, fminX), minY = max(bminY, fminY);
                 const int maxX = min(bmaxX - 1, fmaxX), maxY = min(bmaxY - 1, fmaxY);
                 minX -= minX % 2;
                 minY -= minY % 2;
                 if (qx >= minX && qx <= maxX && qy >= minY && qy <= maxY)
-                    quad_depth<kMS>(t, qx, qy, true, tminX, tminY, keys, sp);
+                    quad_depth<kMS, false>(t, qx, qy, true, tminX, tminY, keys, sp);
             }
         }
     }
@@ -921,18 +961,71 @@ __device__ __forceinline__ RTri broadcast_rtri(const RTri& t, int l) {
     return u;
 }
 
+// Wide references, lane by lane in t (quads: a quad-walked one's number of
+// quads, from pixel (fx, fy), fnx to a row): each by the whole wave, the owner
+// lane's record broadcast with readlane (no memory round trip).
+template <bool kMS>
+__device__ __forceinline__ void walk_wide(const FrameParams& P, const RTri& t, uint32_t pay, bool large, uint32_t quads,
+                                          int fx, int fy, int fnx, int tminX, int tminY, int tmaxX, int tmaxY,
+                                          uint64_t* keys, const SamplePass& sp) {
+    const uint32_t lane = __lane_id();
+    // FineRasterize's quads (bbox clamped to the tile, Core/Rasterizer.h:126-200), 64 per pass
+    uint64_t wm = __ballot(quads != 0);
+    while (wm) {
+        const int l = __ffsll((unsigned long long)wm) - 1;
+        wm &= wm - 1;
+        const RTri u = broadcast_rtri(t, l);
+        const int ux = __builtin_amdgcn_readlane(fx, l), uy = __builtin_amdgcn_readlane(fy, l);
+        const uint32_t unx = __builtin_amdgcn_readlane((uint32_t)fnx, l);
+        const uint32_t uq = __builtin_amdgcn_readlane(quads, l);
+        // quad k = lane + 64 i at (k % unx, k / unx), stepped per pass
+        uint32_t cx = lane % unx, cy = lane / unx;
+        const uint32_t dx = kWave % unx, dy = kWave / unx;
+        for (uint32_t k = lane; k < uq; k += kWave) {
+            quad_depth<kMS, false>(u, ux + 2 * (int)cx, uy + 2 * (int)cy, true, tminX, tminY, keys, sp);
+            cx += dx;
+            cy += dy;
+            if (cx >= unx) {
+                cx -= unx;
+                cy++;
+            }
+        }
+    }
+    uint64_t lm = __ballot(large);
+    while (lm) {
+        const int l = __ffsll((unsigned long long)lm) - 1;
+        lm &= lm - 1;
+        const uint32_t ppay = __builtin_amdgcn_readlane(pay, l);
+        raster_large_wave<kMS>(P, broadcast_rtri(t, l), ppay, tminX, tminY, tmaxX, tmaxY, keys, sp);
+    }
+}
+
+// An item's references that take a whole wave (tile-level ones, and those of
+// kWaveQuads quads or more), by their place in the item: listed while the
+// slices are walked, kWideRefs of them at most at a time, then shared out over
+// the workgroup's waves.  (Not in a direct frame's tiles: few references, spread
+// thinly over the waves anyway, whose records would be loaded twice.)
+template <bool kMS>
+constexpr uint32_t kWideRefs = kMS ? 512 : 1024;  // (a multiple of every workgroup's threads)
+template <bool kMS>
+struct WideRefs {
+    uint32_t n;
+    uint16_t at[kWideRefs<kMS>];
+};
+
 // One raster work item: references [seg << segLog2, (seg + 1) << segLog2) of
-// a tile, segLog2 being the tile's (tile_item).  Each wave streams its own 64-reference slices through the tile's LDS
-// key buffer (no workgroup barrier per slice): small triangles take one lane
-// each, medium ones one quad per lane, tile-level ones the whole wave.  The
-// item's keys go to partials[workIndex].
+// a tile, segLog2 being the tile's (tile_item).  Each wave streams its own
+// 64-reference slices through the tile's LDS key buffer (no workgroup barrier
+// per slice): small triangles take one lane each, medium ones one quad per lane;
+// tile-level and long ones, a whole wave each, are listed and shared out over the
+// waves after the slices.  The item's keys go to partials[workIndex].
 // kThreads: the workgroup's threads.  kDirect: workIndex is a tile of a direct
 // frame with directRefs references, whose keys stay in LDS.
 template <bool kMS, uint32_t kThreads = kBlock, bool kDirect = false>
 __device__ __forceinline__ void raster_item(const BatchParams& Q, const FrameParams* __restrict__ jobs,
                                             const DeviceBuffers& B, uint32_t workIndex,
                                             uint64_t* keys, uint16_t (*sOwner)[kOwnerCap],
-                                            uint32_t directRefs = 0) {
+                                            WideRefs<kMS>* wide, uint32_t directRefs = 0) {
     const uint32_t workItem = kDirect ? workIndex : __builtin_amdgcn_readfirstlane(B.work[workIndex]);
     // segFlag: the segment index, with kSingleSegment >> kTileBits above it
     const uint32_t gtile = workItem & (kMaxBatchTiles - 1), segFlag = workItem >> kTileBits;
@@ -952,8 +1045,11 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
     // item's references once per group of samples.
     const uint32_t S = kMS ? P.samples : 1u;
     for (uint32_t pass = 0; pass * kPassSamples < S; pass++) {
-        const SamplePass sp{P.sample_level, pass * kPassSamples, min(S - pass * kPassSamples, kPassSamples)};
+        const SamplePass sp = kMS ? sample_pass(P.sample_level, pass * kPassSamples,
+                                                min(S - pass * kPassSamples, kPassSamples))
+                                  : SamplePass{1u, 0u};
         for (uint32_t i = threadIdx.x; i < sp.n * kKeyPlane<kMS>; i += kThreads) keys[i] = bg_key();
+        if (!kDirect && threadIdx.x == 0) wide->n = 0;
         __syncthreads();
 
         // Each wave takes slices of L references (64, or a quarter of a short
@@ -967,151 +1063,178 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
         const uint32_t stride = L * (kThreads / kWave);
         const uint32_t first = segBegin + wave * L + lane;
         const uint32_t* segRefs = B.refs + start;
-        auto sv_of = [&](uint32_t pay, const uint3& idx, ScreenVert& a, ScreenVert& b2, ScreenVert& c) {
-            const uint32_t rid = pay & kRecordMask;
-            const bool compact = !(pay >> 31) && rid < Q.total_slots;
-            a = B.sverts[P.vert_base + (compact ? idx.x : 0u)];
-            b2 = B.sverts[P.vert_base + (compact ? idx.y : 0u)];
-            c = B.sverts[P.vert_base + (compact ? idx.z : 0u)];
+        // (An unused index may be anything; a used one is of a checked triangle.)
+        const uint32_t lastV = P.num_vertices - 1u;
+        auto sv_of = [&](const uint3& idx, ScreenVert& a, ScreenVert& b2, ScreenVert& c) {
+            a = B.sverts[P.vert_base + min(idx.x, lastV)];
+            b2 = B.sverts[P.vert_base + min(idx.y, lastV)];
+            c = B.sverts[P.vert_base + min(idx.z, lastV)];
         };
         uint32_t pay1 = segRefs[min(first, segEnd - 1)];
         uint32_t pay2 = segRefs[min(first + stride, segEnd - 1)];
         uint32_t pay3 = segRefs[min(first + 2 * stride, segEnd - 1)];
         ScreenVert n0, n1, n2;
-        sv_of(pay1, ref_indices(P, Q.total_slots, pay1), n0, n1, n2);
-        uint3 idx2 = ref_indices(P, Q.total_slots, pay2);
-        for (uint32_t b = segBegin + wave * L; b < segEnd; b += stride) {
-            const uint32_t p = b + lane;
-            const bool valid = lane < L && p < segEnd;
-            const uint32_t pay = pay1;
-            const uint32_t rid = pay & kRecordMask;
-            const bool trivial = ((pay >> kRecordBits) & 7u) == 7u;
-            const bool big = (pay >> 31) != 0;
-            const bool compact = !big && rid < Q.total_slots;
-            const ScreenVert s0 = n0, s1 = n1, s2 = n2;
-            sv_of(pay2, idx2, n0, n1, n2);
-            idx2 = ref_indices(P, Q.total_slots, pay3);
-            pay1 = pay2;
-            pay2 = pay3;
-            pay3 = segRefs[min(p + 3 * stride, segEnd - 1)];
-            // Tile-level paths (RasterizeTile, Core/Renderer.cpp:255-268):
-            // trivially accepted, or big with hierarchical rasterisation on.
-            const bool large = valid && (trivial || (big && P.hierarchical));
-            // Every lane holds its own record; large ones are broadcast below.
-            RTri t;
-            screen_rtri_from(s0, s1, s2, rid, t);
-            if (valid && !compact) load_rtri(B.rrec[rid], t);
-            uint32_t myQ = 0;  // quads of a FineRasterize reference beyond the tiny path
-            int fx = 0, fy = 0, fnx = 1;
-            if (valid && !large) {
-                const int bx0 = min(t.x0, min(t.x1, t.x2)) >> 4, bx1 = max(t.x0, max(t.x1, t.x2)) >> 4;
-                const int by0 = min(t.y0, min(t.y1, t.y2)) >> 4, by1 = max(t.y0, max(t.y1, t.y2)) >> 4;
-                // FineRasterize_SingleSample bbox (Core/Rasterizer.h:132-140).
-                int minX = max(tminX, bx0);
-                const int maxX = min(tmaxX - 1, bx1);
-                int minY = max(tminY, by0);
-                const int maxY = min(tmaxY - 1, by1);
-                if (bx1 - bx0 <= 1 && by1 - by0 <= 1) {
-                    // Pixel bbox of at most 2x2: test only its pixels.  The
-                    // reference's even-aligned quads add pixels whose centres lie
-                    // outside the bbox, hence outside the triangle, and with edges
-                    // this short no edge function can wrap.
-                    if (maxX >= minX && maxY >= minY)
-                        quad_depth<kMS>(t, minX, minY, true, tminX, tminY, keys, maxX, maxY, sp);
-                } else {
-                    minX -= minX % 2;
-                    minY -= minY % 2;
-                    if (maxX >= minX && maxY >= minY) {
-                        const int nqx = (maxX - minX) / 2 + 1, nqy = (maxY - minY) / 2 + 1;
-                        myQ = (uint32_t)(nqx * nqy);
-                        fx = minX;
-                        fy = minY;
-                        fnx = nqx;
+        sv_of(ref_indices(P, pay1), n0, n1, n2);
+        uint3 idx2 = ref_indices(P, pay2);
+        // Pixel box of a FineRasterize reference (Core/Rasterizer.h:132-140);
+        // whether the triangle's own is at most 2x2.
+        auto pixel_box = [&](const RTri& t, int& minX, int& maxX, int& minY, int& maxY) {
+            const int bx0 = min(t.x0, min(t.x1, t.x2)) >> 4, bx1 = max(t.x0, max(t.x1, t.x2)) >> 4;
+            const int by0 = min(t.y0, min(t.y1, t.y2)) >> 4, by1 = max(t.y0, max(t.y1, t.y2)) >> 4;
+            minX = max(tminX, bx0);
+            maxX = min(tmaxX - 1, bx1);
+            minY = max(tminY, by0);
+            maxY = min(tmaxY - 1, by1);
+            return bx1 - bx0 <= 1 && by1 - by0 <= 1;
+        };
+        // Quads of a reference beyond the tiny path: the first one's pixel, quads per row.
+        auto quad_box = [&](int minX, int maxX, int minY, int maxY, int& fx, int& fy, int& fnx) -> uint32_t {
+            minX &= ~1;
+            minY &= ~1;
+            if (maxX < minX || maxY < minY) return 0;
+            fx = minX;
+            fy = minY;
+            fnx = (int)((uint32_t)(maxX - minX) / 2u) + 1;
+            return (uint32_t)fnx * ((uint32_t)(maxY - minY) / 2u + 1u);
+        };
+        uint32_t b = segBegin + wave * L;
+        for (uint32_t until = kDirect ? segEnd : segBegin + kWideRefs<kMS>;; until += kWideRefs<kMS>) {
+            for (; b < min(segEnd, until); b += stride) {
+                const uint32_t p = b + lane;
+                const bool valid = lane < L && p < segEnd;
+                const uint32_t pay = pay1;
+                const uint32_t rid = pay & kRecordMask;
+                const bool trivial = ((pay >> kRecordBits) & 7u) == 7u;
+                const bool big = (pay >> 31) != 0;
+                const bool compact = !big && rid < Q.total_slots;
+                const ScreenVert s0 = n0, s1 = n1, s2 = n2;
+                sv_of(idx2, n0, n1, n2);
+                idx2 = ref_indices(P, pay3);
+                pay1 = pay2;
+                pay2 = pay3;
+                pay3 = segRefs[min(p + 3 * stride, segEnd - 1)];
+                // Tile-level paths (RasterizeTile, Core/Renderer.cpp:255-268):
+                // trivially accepted, or big with hierarchical rasterisation on.
+                const bool large = valid && (trivial || (big && P.hierarchical));
+                // Every lane holds its own record; large ones are broadcast below.
+                RTri t;
+                screen_rtri_from(s0, s1, s2, rid, t);
+                bool fits = true;
+                if (valid && !compact) {
+                    load_rtri(B.rrec[rid], t);
+                    fits = fits24(t);
+                }
+                uint32_t myQ = 0;  // quads of a FineRasterize reference beyond the tiny path
+                int fx = 0, fy = 0, fnx = 1;
+                if (valid && !large) {
+                    int minX, maxX, minY, maxY;
+                    if (pixel_box(t, minX, maxX, minY, maxY)) {
+                        // Test only the box's pixels.  The reference's even-aligned
+                        // quads add pixels whose centres lie outside the bbox, hence
+                        // outside the triangle, and with edges this short no edge
+                        // function can wrap.
+                        if (maxX >= minX && maxY >= minY)
+                            quad_depth<kMS, true>(t, minX, minY, true, tminX, tminY, keys, maxX, maxY, sp);
+                    } else {
+                        myQ = quad_box(minX, maxX, minY, maxY, fx, fy, fnx);
                     }
                 }
-            }
-            // Medium references of kWaveQuads quads or more: the whole wave walks
-            // each one's FineRasterize quads (bbox clamped to the tile,
-            // Core/Rasterizer.h:126-200), 64 per pass.
-            uint64_t wm = __ballot(myQ >= kWaveQuads);
-            while (wm) {
-                const int l = __ffsll((unsigned long long)wm) - 1;
-                wm &= wm - 1;
-                const RTri u = broadcast_rtri(t, l);
-                const int ux = __builtin_amdgcn_readlane(fx, l), uy = __builtin_amdgcn_readlane(fy, l);
-                const uint32_t unx = __builtin_amdgcn_readlane((uint32_t)fnx, l);
-                const uint32_t uq = __builtin_amdgcn_readlane(myQ, l);
-                // quad k = lane + 64 i at (k % unx, k / unx), stepped per pass
-                uint32_t cx = lane % unx, cy = lane / unx;
-                const uint32_t dx = kWave % unx, dy = kWave / unx;
-                for (uint32_t k = lane; k < uq; k += kWave) {
-                    quad_depth<kMS>(u, ux + 2 * (int)cx, uy + 2 * (int)cy, true, tminX, tminY, keys, sp);
-                    cx += dx;
-                    cy += dy;
-                    if (cx >= unx) {
-                        cx -= unx;
-                        cy++;
-                    }
+                const bool isWide = large || myQ >= kWaveQuads || (myQ && !fits);
+                if (kDirect) {
+                    walk_wide<kMS>(P, t, pay, large, isWide ? myQ : 0u, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY,
+                                   keys, sp);
+                } else if (const uint64_t wm = __ballot(isWide)) {
+                    uint32_t at = 0;
+                    if (lane == 0) at = atomicAdd(&wide->n, (uint32_t)__popcll(wm));
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    if (isWide) wide->at[at + (uint32_t)__popcll(wm & lanemask_lt())] = (uint16_t)(p - segBegin);
                 }
-            }
-            if (myQ >= kWaveQuads) myQ = 0;
-            // Other references with quads: the wave's quads are expanded into
-            // (reference, quad) pairs and tested 64 per pass, one quad per lane.
-            // Pair k's entry in the wave's owner table holds the owner lane and
-            // the quad's column and row in the owner's bbox.
-            const uint32_t incl = wave_incl_scan(myQ);
-            const uint32_t totalQ = __builtin_amdgcn_readlane(incl, kWave - 1);
-            if (totalQ) {
-                {
-                    uint16_t* own = &sOwner[wave][incl - myQ];
-                    uint32_t cx = 0, cy = 0;
-                    for (uint32_t i = 0; __ballot(i < myQ); i++) {
-                        if (i < myQ) {
-                            own[i] = (uint16_t)(lane | (cx << 6) | (cy << 10));
-                            if (++cx == (uint32_t)fnx) {
-                                cx = 0;
-                                cy++;
+                if (isWide) myQ = 0;
+                // Other references with quads: the wave's quads are expanded into
+                // (reference, quad) pairs and tested 64 per pass, one quad per lane.
+                // Pair k's entry in the wave's owner table holds the owner lane and
+                // the quad's column and row in the owner's bbox.
+                const uint32_t incl = wave_incl_scan(myQ);
+                const uint32_t totalQ = __builtin_amdgcn_readlane(incl, kWave - 1);
+                if (totalQ) {
+                    {
+                        uint16_t* own = &sOwner[wave][incl - myQ];
+                        uint32_t cx = 0, cy = 0;
+                        for (uint32_t i = 0; __ballot(i < myQ); i++) {
+                            if (i < myQ) {
+                                own[i] = (uint16_t)(lane | (cx << 6) | (cy << 10));
+                                if (++cx == (uint32_t)fnx) {
+                                    cx = 0;
+                                    cy++;
+                                }
                             }
                         }
                     }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                for (uint32_t base = 0; base < totalQ; base += kWave) {
-                    const uint32_t k = base + lane;
-                    const uint32_t e = k < totalQ ? sOwner[wave][k] : 0u;
-                    const int j = (int)(e & 63u);
-                    RTri u;
-                    u.x0 = __shfl(t.x0, j); u.y0 = __shfl(t.y0, j);
-                    u.x1 = __shfl(t.x1, j); u.y1 = __shfl(t.y1, j);
-                    u.x2 = __shfl(t.x2, j); u.y2 = __shfl(t.y2, j);
-                    u.B0 = u.y0 - u.y1; u.C0 = u.x1 - u.x0;
-                    u.B1 = u.y1 - u.y2; u.C1 = u.x2 - u.x1;
-                    u.B2 = u.y2 - u.y0; u.C2 = u.x0 - u.x2;
-                    u.pb0 = __shfl(t.pb0, j); u.pb1 = __shfl(t.pb1, j); u.pb2 = __shfl(t.pb2, j);
-                    u.inv_det = __shfl(t.inv_det, j);
-                    u.z0 = __shfl(t.z0, j); u.z1 = __shfl(t.z1, j); u.z2 = __shfl(t.z2, j);
-                    u.order = __shfl(t.order, j);
-                    const int ux = __shfl(fx, j), uy = __shfl(fy, j);
-                    if (k < totalQ)
-                        quad_depth<kMS>(u, ux + 2 * (int)((e >> 6) & 15u), uy + 2 * (int)(e >> 10), true, tminX,
-                                        tminY, keys, sp);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    for (uint32_t base = 0; base < totalQ; base += kWave) {
+                        const uint32_t k = base + lane;
+                        const uint32_t e = k < totalQ ? sOwner[wave][k] : 0u;
+                        const int j = (int)(e & 63u);
+                        RTri u;
+                        u.x0 = __shfl(t.x0, j); u.y0 = __shfl(t.y0, j);
+                        u.x1 = __shfl(t.x1, j); u.y1 = __shfl(t.y1, j);
+                        u.x2 = __shfl(t.x2, j); u.y2 = __shfl(t.y2, j);
+                        u.B0 = u.y0 - u.y1; u.C0 = u.x1 - u.x0;
+                        u.B1 = u.y1 - u.y2; u.C1 = u.x2 - u.x1;
+                        u.B2 = u.y2 - u.y0; u.C2 = u.x0 - u.x2;
+                        u.pb0 = __shfl(t.pb0, j); u.pb1 = __shfl(t.pb1, j); u.pb2 = __shfl(t.pb2, j);
+                        u.inv_det = __shfl(t.inv_det, j);
+                        u.z0 = __shfl(t.z0, j); u.z1 = __shfl(t.z1, j); u.z2 = __shfl(t.z2, j);
+                        u.order = __shfl(t.order, j);
+                        const int ux = __shfl(fx, j), uy = __shfl(fy, j);
+                        if (k < totalQ)
+                            quad_depth<kMS, true>(u, ux + 2 * (int)((e >> 6) & 15u), uy + 2 * (int)(e >> 10), true,
+                                                  tminX, tminY, keys, sp);
+                    }
                 }
             }
-            // Large references: the whole wave takes them one at a time, the
-            // owner lane's record broadcast with readlane (no memory round trip).
-            uint64_t lm = __ballot(large);
-            while (lm) {
-                const int l = __ffsll((unsigned long long)lm) - 1;
-                lm &= lm - 1;
-                const uint32_t ppay = __builtin_amdgcn_readlane(pay, l);
-                raster_large_wave<kMS>(P, broadcast_rtri(t, l), ppay, tminX, tminY, tmaxX, tmaxY, keys, sp);
+            __syncthreads();
+            if (kDirect) return;
+            // The listed references, dealt out to the waves.  (When each wave
+            // walked its own slices' wide references, the wave that had the item's
+            // last slice walked most of them, as heavy references end a tile's
+            // list: 12 quad-walked and 10 tile-level ones made an item of 39 us
+            // beside 12 on average, and the 2.1M sphere grid at 1080p took 45 us,
+            // 127 with 4 samples; so 36 and 86.  With a quadrant or 64 quads of each
+            // reference per wave its preparation by four waves cost more than the
+            // finer split gave: 40 and 86.)
+            const uint32_t nWide = __builtin_amdgcn_readfirstlane(wide->n);
+            for (uint32_t e0 = 0; e0 < nWide; e0 += kThreads) {
+                const uint32_t e = e0 + wave + kThreads / kWave * lane;
+                const bool valid = e < nWide;
+                const uint32_t pay = segRefs[segBegin + wide->at[valid ? e : 0u]];
+                const uint32_t rid = pay & kRecordMask;
+                const bool big = (pay >> 31) != 0, trivial = ((pay >> kRecordBits) & 7u) == 7u;
+                const bool large = valid && (trivial || (big && P.hierarchical));
+                RTri t;
+                if (big || rid >= Q.total_slots) load_rtri(B.rrec[rid], t);
+                else screen_rtri(P, B, rid, t);
+                uint32_t quads = 0;
+                int fx = 0, fy = 0, fnx = 1;
+                if (valid && !large) {
+                    int minX, maxX, minY, maxY;
+                    pixel_box(t, minX, maxX, minY, maxY);
+                    quads = quad_box(minX, maxX, minY, maxY, fx, fy, fnx);
+                }
+                walk_wide<kMS>(P, t, pay, large, quads, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY, keys, sp);
             }
+            if (until >= segEnd) {
+                if (nWide) __syncthreads();
+                break;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) wide->n = 0;
+            __syncthreads();
         }
-        __syncthreads();
-        if (kDirect) return;
-        uint64_t* g = B.partials + ((size_t)((tileItem & kImageMask) + seg) * S + sp.base) * (kTileSize * kTileSize);
+        uint64_t* g = B.partials +
+                      ((size_t)((tileItem & kImageMask) + seg) * S + pass * kPassSamples) * (kTileSize * kTileSize);
         // A tile of one segment has no other image to merge with, and k_shade
         // recomputes the depth: the low words of the keys (the winners'
         // orders; 0xFFFFFFFF where nothing was drawn) are its image.
@@ -1166,7 +1289,7 @@ __device__ __forceinline__ void winner_tri(const FrameParams& P, const DeviceBuf
         v2 = B.verts[s.v2];
         load_rtri(B.rrec[ri], t);
     } else {
-        const uint32_t* idx = P.mesh.idx + 3 * (size_t)(tri - P.slot_base);
+        const GlobalPtr<uint32_t> idx = as_global(P.mesh.idx) + 3 * (size_t)(tri - P.slot_base);
         const uint32_t v0i = P.vert_base + idx[0], v1i = P.vert_base + idx[1], v2i = P.vert_base + idx[2];
         if (recompute) {
             v0 = B.verts[v0i];

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kTileThreads, kTex ? 4 : 6) void k_tile(BatchParams
     const uint32_t tile = gtile - P.tile_base;
     const int tminX = (int)(tile % P.tiles_x) * kTileSize, tminY = (int)(tile / P.tiles_x) * kTileSize;
     const int tmaxX = min(tminX + kTileSize, (int)P.width), tmaxY = min(tminY + kTileSize, (int)P.height);
-    raster_item<false, kTileThreads, true>(Q, jobs, B, gtile, keys, sOwner, n);
+    raster_item<false, kTileThreads, true>(Q, jobs, B, gtile, keys, sOwner, nullptr, n);
     for (uint32_t i = threadIdx.x; i < kTileSize * kTileSize; i += kTileThreads) {
         const int x = tminX + (int)(i % kTileSize), y = tminY + (int)(i / kTileSize);
         if (x >= tmaxX || y >= tmaxY) continue;

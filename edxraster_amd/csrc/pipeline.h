@@ -69,6 +69,7 @@ constexpr uint32_t kDescCompact = 1u << 31;
 // or more pixels (it takes a whole wave in the raster; counted in tile_big).
 constexpr uint32_t kDescHeavy = 1u << 30;
 constexpr uint32_t kHeavyPixels = 256;
+constexpr uint32_t kCompactExtent = 1u << 14;  // of a compact triangle's bounding box, in 1/16 pixels
 
 enum ShaderKind { kLambertAlbedo = 0, kBlinnPhongRef = 1, kVcBlinnPhong = 2, kTexturedLambert = 3 };
 enum TextureFilter {

@@ -303,18 +303,18 @@ constexpr uint32_t kClipWaves = 16;  // waves (triangles) per workgroup pass
 // Input vertex v of a job's mesh with its shading attributes (the caller sets inv_w).
 __device__ __forceinline__ ShadeVert input_vertex(const MeshPtrs& M, uint32_t v) {
     ShadeVert o;
-    o.px = M.px[v];
-    o.py = M.py[v];
-    o.pz = M.pz[v];
-    o.nx = M.nx[v];
-    o.ny = M.ny[v];
-    o.nz = M.nz[v];
-    o.cr = M.cr ? M.cr[v] : 0.0f;
-    o.cg = M.cg ? M.cg[v] : 0.0f;
-    o.cb = M.cb ? M.cb[v] : 0.0f;
+    o.px = global_at(M.px, v);
+    o.py = global_at(M.py, v);
+    o.pz = global_at(M.pz, v);
+    o.nx = global_at(M.nx, v);
+    o.ny = global_at(M.ny, v);
+    o.nz = global_at(M.nz, v);
+    o.cr = M.cr ? global_at(M.cr, v) : 0.0f;
+    o.cg = M.cg ? global_at(M.cg, v) : 0.0f;
+    o.cb = M.cb ? global_at(M.cb, v) : 0.0f;
     o.inv_w = 0.0f;
-    o.u = M.tu ? M.tu[v] : 0.0f;
-    o.v = M.tv ? M.tv[v] : 0.0f;
+    o.u = M.tu ? global_at(M.tu, v) : 0.0f;
+    o.v = M.tv ? global_at(M.tv, v) : 0.0f;
     return o;
 }
 }  // namespace
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(kClipWaves * 64) void k_clip(BatchParams Q, const F
             t = __builtin_amdgcn_readfirstlane(B.clip_queue[q]);  // triangle slot
             Pp = &jobs[Q.num_jobs == 1 ? 0u : __builtin_amdgcn_readfirstlane(Q.sblock_job[t / kBlock])];
             const FrameParams& P = *Pp;
-            const uint32_t* idx = P.mesh.idx + 3 * (size_t)(t - P.slot_base);
+            const GlobalPtr<uint32_t> idx = as_global(P.mesh.idx) + 3 * (size_t)(t - P.slot_base);
             vi[0] = P.vert_base + __builtin_amdgcn_readfirstlane(idx[0]);
             vi[1] = P.vert_base + __builtin_amdgcn_readfirstlane(idx[1]);
             vi[2] = P.vert_base + __builtin_amdgcn_readfirstlane(idx[2]);
@@ -1340,12 +1340,17 @@ __global__ __launch_bounds__(kBlock) void k_bin_scatter(BatchParams Q, const Fra
 // Persistent raster kernel: workgroups pull (tile, segment) items from the
 // list built by k_bin_tilescan until it is exhausted.  The single-sample
 // kernel is held to 96 VGPRs so that five workgroups per CU, as many as its LDS
-// allows, are resident.
+// allows, are resident.  The multisample kernel's key planes take 32 KB, so that
+// waves, not workgroups, are made more: two workgroups of eight waves per CU
+// (2.1M sphere grid at 1080p, 4 samples: 92 us with three of four waves, so 88).
 template <bool kMS>
-__global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, const FrameParams* __restrict__ jobs,
+constexpr uint32_t kRasterThreads = kMS ? 2 * kBlock : kBlock;
+template <bool kMS>
+__global__ __launch_bounds__(kRasterThreads<kMS>, kMS ? 4 : 5) void k_raster(BatchParams Q, const FrameParams* __restrict__ jobs,
                                                    DeviceBuffers B) {
     __shared__ uint64_t keys[(kMS ? kPassSamples : 1) * kKeyPlane<kMS>];
-    __shared__ uint16_t sOwner[kBlock / kWave][kOwnerCap];
+    __shared__ uint16_t sOwner[kRasterThreads<kMS> / kWave][kOwnerCap];
+    __shared__ WideRefs<kMS> sWide;
     __shared__ uint32_t sItem;
     // The counters are final (this kernel only draws items from kCntWorkNext):
     // the last workgroup, which in small frames has no item, copies them to
@@ -1354,7 +1359,7 @@ __global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, c
     // launch of its own after the frame took 4 us and the gap before it, and
     // a copy queued behind the frame 12 us.
     if (blockIdx.x == gridDim.x - 1)
-        for (uint32_t i = threadIdx.x; i < kCntSlots; i += kBlock) B.host_counters[i] = B.counters[i];
+        for (uint32_t i = threadIdx.x; i < kCntSlots; i += kRasterThreads<kMS>) B.host_counters[i] = B.counters[i];
     if (B.counters[kCntOverflow] & kOvNoLists) return;
     const uint32_t nItems = B.counters[kCntWorkItems];
     // Single-sample batches: the empty tiles are cleared here, a share per
@@ -1369,7 +1374,7 @@ __global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, c
             while (m) {
                 const uint32_t l = (uint32_t)__ffsll((unsigned long long)m) - 1;
                 m &= m - 1;
-                clear_tile<kBlock>(Q, jobs, B, base + l * gridDim.x);
+                clear_tile<kRasterThreads<kMS>>(Q, jobs, B, base + l * gridDim.x);
             }
         }
     }
@@ -1380,7 +1385,7 @@ __global__ __launch_bounds__(kBlock, kMS ? 3 : 5) void k_raster(BatchParams Q, c
         __syncthreads();
         const uint32_t item = __builtin_amdgcn_readfirstlane(sItem);
         if (item >= nItems) break;
-        raster_item<kMS>(Q, jobs, B, item, keys, sOwner);
+        raster_item<kMS, kRasterThreads<kMS>>(Q, jobs, B, item, keys, sOwner, &sWide);
         __syncthreads();
     }
 }
@@ -1580,7 +1585,8 @@ hipError_t init_kernels() {
                                                          reinterpret_cast<const void*>(&k_raster<false>), kBlock, 0);
     if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&g_rasterResident[1],
-                                                         reinterpret_cast<const void*>(&k_raster<true>), kBlock, 0);
+                                                         reinterpret_cast<const void*>(&k_raster<true>),
+                                                         kRasterThreads<true>, 0);
     return e;
 }
 
@@ -1701,7 +1707,7 @@ hipError_t launch_frame(const BatchParams& Q, FrameParams* jobs, const FramePara
     mark(3);
     if (Q.total_chunks) hipLaunchKernelGGL(k_bin_scatter, dim3(Q.total_chunks), dim3(kBlock), lds, s, Q, jobs, B);
     mark(4);
-    if (Q.max_samples > 1) hipLaunchKernelGGL((k_raster<true>), dim3(B.raster_grid), dim3(kBlock), 0, s, Q, jobs, B);
+    if (Q.max_samples > 1) hipLaunchKernelGGL((k_raster<true>), dim3(B.raster_grid), dim3(kRasterThreads<true>), 0, s, Q, jobs, B);
     else hipLaunchKernelGGL((k_raster<false>), dim3(B.raster_grid), dim3(kBlock), 0, s, Q, jobs, B);
     const dim3 shadeThreads(kShadeThreads);
     auto shade = [&](auto plain, auto textured, dim3 grid) {
