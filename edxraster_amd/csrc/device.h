@@ -1249,14 +1249,34 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
     }
 }
 
-// Cleared pixels of an empty tile (as k_shade writes uncovered ones).
+// Cleared pixels of an empty tile (as k_shade writes uncovered ones): four pixels
+// per store where the rows start on 16 bytes, else one.  thread: of kThreads that
+// share the tile.
 template <uint32_t kThreads>
 __device__ __forceinline__ void clear_tile(const BatchParams& Q, const FrameParams* __restrict__ jobs,
-                                           const DeviceBuffers& B, uint32_t gtile) {
+                                           const DeviceBuffers& B, uint32_t gtile, uint32_t thread) {
     const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];
     const uint32_t tile = gtile - P.tile_base;
     const int tminX = (int)(tile % P.tiles_x) * kTileSize, tminY = (int)(tile / P.tiles_x) * kTileSize;
-    for (uint32_t i = threadIdx.x; i < kTileSize * kTileSize; i += kThreads) {
+    const uint64_t align = (uint64_t)B.color | (uint64_t)B.depth | (uint64_t)B.ids | (uint64_t)B.color_f32 |
+                           4ull * (P.pix_base | P.width);
+    if (!(align & 15u)) {
+        constexpr uint32_t kRow = kTileSize / 4;
+        for (uint32_t i = thread; i < kRow * kTileSize; i += kThreads) {
+            const int x = tminX + (int)(i % kRow) * 4, y = tminY + (int)(i / kRow);
+            if (x < (int)P.width && y < (int)P.height) {
+                const size_t o = P.pix_base + (size_t)(P.height - 1 - y) * P.width + x;
+                *reinterpret_cast<uint4*>(B.color + o) = make_uint4(0u, 0u, 0u, 0u);
+                *reinterpret_cast<float4*>(B.depth + o) = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                *reinterpret_cast<uint4*>(B.ids + o) = make_uint4(~0u, ~0u, ~0u, ~0u);
+                if (B.color_f32)
+                    for (uint32_t k = 0; k < 3; k++)
+                        reinterpret_cast<float4*>(B.color_f32 + 3 * o)[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
+        return;
+    }
+    for (uint32_t i = thread; i < kTileSize * kTileSize; i += kThreads) {
         const int x = tminX + (int)(i % kTileSize), y = tminY + (int)(i / kTileSize);
         if (x < (int)P.width && y < (int)P.height) {
             const size_t o = P.pix_base + (size_t)(P.height - 1 - y) * P.width + x;

@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kTileThreads, kTex ? 4 : 6) void k_tile(BatchParams
     __syncthreads();
     const uint32_t n = __builtin_amdgcn_readfirstlane(sCount);
     if (!n) {
-        clear_tile<kTileThreads>(Q, jobs, B, gtile);
+        clear_tile<kTileThreads>(Q, jobs, B, gtile, threadIdx.x);
         return;
     }
     const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];

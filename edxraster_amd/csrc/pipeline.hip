@@ -1345,6 +1345,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_scatter(BatchParams Q, const Fra
 // (2.1M sphere grid at 1080p, 4 samples: 92 us with three of four waves, so 88).
 template <bool kMS>
 constexpr uint32_t kRasterThreads = kMS ? 2 * kBlock : kBlock;
+// References that clearing an empty tile counts as (k_raster), without and with float colours.
+constexpr uint32_t kClearRefs = 16, kClearRefsFloat = 128;
 template <bool kMS>
 __global__ __launch_bounds__(kRasterThreads<kMS>, kMS ? 4 : 5) void k_raster(BatchParams Q, const FrameParams* __restrict__ jobs,
                                                    DeviceBuffers B) {
@@ -1362,19 +1364,37 @@ __global__ __launch_bounds__(kRasterThreads<kMS>, kMS ? 4 : 5) void k_raster(Bat
         for (uint32_t i = threadIdx.x; i < kCntSlots; i += kRasterThreads<kMS>) B.host_counters[i] = B.counters[i];
     if (B.counters[kCntOverflow] & kOvNoLists) return;
     const uint32_t nItems = B.counters[kCntWorkItems];
-    // Single-sample batches: the empty tiles are cleared here, a share per
-    // workgroup, before any item is taken (k_shade skips them).  Lane l looks
-    // at tile blockIdx.x + l * gridDim.x of each pass; every wave computes the
-    // same mask.
-    if (!kMS) {
-        for (uint32_t base = blockIdx.x; base < Q.total_tiles; base += gridDim.x * kWave) {
-            const uint32_t t = base + __lane_id() * gridDim.x;
-            const bool empty = t < Q.total_tiles && B.tile_start[t + 1] == B.tile_start[t];
+    // Single-sample frames and batches: the empty tiles are cleared here (k_shade
+    // skips them), by the waves of the last workgroups before these take an item,
+    // while the others rasterise: the clears are bound by stores, the items by the
+    // ALU.  With a share of the clears at the head of every workgroup nothing
+    // overlapped: 256 jobs 630 us, so 515 (117K tiles, two thirds of them empty).
+    // The clearing workgroups are the share that clearing has of the work, a tile
+    // weighing as many references as below, and a tenth at least, which deep tiles
+    // of many items among empty ones need.  256 jobs with a weight of 16, 32, 64:
+    // 518, 538, 555 us.  With float colours, twice the bytes and few references per
+    // tile (64 views at 512): 104, 106, 98 us with 32, 64, 128 (97 before).
+    // A wave looks at tiles base + lane * step of each pass.  (The four waves of a
+    // workgroup on one tile: a tenth of the workgroups then took 706 us for 256
+    // jobs, waiting for each tile's job.)
+    const uint32_t tiles = Q.total_tiles;
+    const float clearing =
+        (float)(tiles - min(tiles, nItems)) * (float)(B.color_f32 ? kClearRefsFloat : kClearRefs);
+    const float share = clearing / (clearing + (float)B.counters[kCntTotalRefs] + 1.0f);
+    const uint32_t clearers =
+        min(gridDim.x, max(gridDim.x / 10, (uint32_t)((float)gridDim.x * share)) + 1);
+    if (!kMS && blockIdx.x + clearers >= gridDim.x) {
+        constexpr uint32_t kWaves = kRasterThreads<kMS> / kWave;
+        const uint32_t step = clearers * kWaves;
+        for (uint32_t base = __builtin_amdgcn_readfirstlane((gridDim.x - 1 - blockIdx.x) * kWaves + threadIdx.x / kWave);
+             base < tiles; base += step * kWave) {
+            const uint32_t t = base + __lane_id() * step;
+            const bool empty = t < tiles && B.tile_start[t + 1] == B.tile_start[t];
             uint64_t m = __ballot(empty);
             while (m) {
                 const uint32_t l = (uint32_t)__ffsll((unsigned long long)m) - 1;
                 m &= m - 1;
-                clear_tile<kRasterThreads<kMS>>(Q, jobs, B, base + l * gridDim.x);
+                clear_tile<kWave>(Q, jobs, B, base + l * step, __lane_id());
             }
         }
     }
