@@ -1553,7 +1553,9 @@ __device__ __forceinline__ void shade_samples(const BatchParams& Q, const FrameP
             B.ids[o + s * plane] = (order >> 4) - P.slot_base;
             rgba = cachedColor;
         }
-        for (int ch = 0; ch < 4; ch++) acc[ch] += (float)((rgba >> (8 * ch)) & 255u) / 255.0f;
+        // (byte / 255, from the rounded 1 / 255)
+        for (int ch = 0; ch < 4; ch++)
+            acc[ch] += quotient_normal((float)((rgba >> (8 * ch)) & 255u), 255.0f, 1.0f / 255.0f);
     }
     const float invS = 1.0f / (float)S;
     B.color[o] = to_byte(acc[0] * invS) | (to_byte(acc[1] * invS) << 8) | (to_byte(acc[2] * invS) << 16) |
