@@ -921,21 +921,21 @@ __device__ __forceinline__ float3 shade_any(const FrameParams& P, const RTri& t,
 namespace {
 
 // Tile-level references for one wave: the lanes are the 8x8 quads of a
-// 16x16-pixel quadrant and the wave walks the tile's four quadrants.  Covers
+// 16x16-pixel quadrant and the wave walks the tile's quadrants q0 .. q1 - 1.  Covers
 // TrivialAcceptTriangle over the tile and CoarseRasterize's stepped quadrant
 // tests with FineRasterize inside partly covered quadrants
 // (Core/Rasterizer.h:32-200,310-353).
 template <bool kMS>
 __device__ __forceinline__ void raster_large_wave(const FrameParams& P, const RTri& t, uint32_t pay,
                                                   int tminX, int tminY, int tmaxX, int tmaxY, uint64_t* keys,
-                                                  const SamplePass& sp) {
+                                                  const SamplePass& sp, int q0, int q1) {
     const uint32_t lane = __lane_id();
     const int lx = (int)(lane & 7u) * 2, ly = (int)(lane >> 3) * 2;
     const bool trivial = ((pay >> kRecordBits) & 7u) == 7u;
     const bool big = (pay >> 31) != 0;
     if (trivial) {
         // TrivialAcceptTriangle over the tile (Core/Rasterizer.h:310-353).
-        for (int q = 0; q < 4; q++) {
+        for (int q = q0; q < q1; q++) {
             const int qx = tminX + 16 * (q & 1) + lx, qy = tminY + 16 * (q >> 1) + ly;
             if (qx <= tmaxX - 1 && qy <= tmaxY - 1) quad_depth<kMS, false>(t, qx, qy, false, tminX, tminY, keys, sp);
         }
@@ -969,7 +969,7 @@ __device__ __forceinline__ void raster_large_wave(const FrameParams& P, const RT
         const int ac0 = ae0 ? 0 : ef(0, a0), ac1 = ae1 ? 0 : ef(1, a1), ac2 = ae2 ? 0 : ef(2, a2);
         const int fminX = min(t.x0, min(t.x1, t.x2)) >> 4, fmaxX = max(t.x0, max(t.x1, t.x2)) >> 4;
         const int fminY = min(t.y0, min(t.y1, t.y2)) >> 4, fmaxY = max(t.y0, max(t.y1, t.y2)) >> 4;
-        for (int q = 0; q < 4; q++) {
+        for (int q = q0; q < q1; q++) {
             const bool rej = (rj0 + step(r0, t.B0, t.C0, q) < 0) || (rj1 + step(r1, t.B1, t.C1, q) < 0) ||
                              (rj2 + step(r2, t.B2, t.C2, q) < 0);
             if (rej) continue;
@@ -1024,7 +1024,7 @@ __device__ __forceinline__ RTri broadcast_rtri(const RTri& t, int l) {
 template <bool kMS>
 __device__ __forceinline__ void walk_wide(const FrameParams& P, const RTri& t, uint32_t pay, bool large, uint32_t quads,
                                           int fx, int fy, int fnx, int tminX, int tminY, int tmaxX, int tmaxY,
-                                          uint64_t* keys, const SamplePass& sp) {
+                                          uint64_t* keys, const SamplePass& sp, int q0 = 0, int q1 = 4) {
     const uint32_t lane = __lane_id();
     // FineRasterize's quads (bbox clamped to the tile, Core/Rasterizer.h:126-200), 64 per pass
     uint64_t wm = __ballot(quads != 0);
@@ -1053,7 +1053,7 @@ __device__ __forceinline__ void walk_wide(const FrameParams& P, const RTri& t, u
         const int l = __ffsll((unsigned long long)lm) - 1;
         lm &= lm - 1;
         const uint32_t ppay = __builtin_amdgcn_readlane(pay, l);
-        raster_large_wave<kMS>(P, broadcast_rtri(t, l), ppay, tminX, tminY, tmaxX, tmaxY, keys, sp);
+        raster_large_wave<kMS>(P, broadcast_rtri(t, l), ppay, tminX, tminY, tmaxX, tmaxY, keys, sp, q0, q1);
     }
 }
 
@@ -1077,12 +1077,14 @@ struct WideRefs {
 // tile-level and long ones, a whole wave each, are listed and shared out over the
 // waves after the slices.  The item's keys go to partials[workIndex].
 // kThreads: the workgroup's threads.  kDirect: workIndex is a tile of a direct
-// frame with directRefs references, whose keys stay in LDS.
+// frame with directRefs references, whose keys stay in LDS, of rows [row0, row1)
+// only (0, 16 or 32).
 template <bool kMS, uint32_t kThreads = kBlock, bool kDirect = false>
 __device__ __forceinline__ void raster_item(const BatchParams& Q, const FrameParams* __restrict__ jobs,
                                             const DeviceBuffers& B, uint32_t workIndex,
                                             uint64_t* keys, uint16_t (*sOwner)[kOwnerCap],
-                                            WideRefs<kMS>* wide, uint32_t directRefs = 0) {
+                                            WideRefs<kMS>* wide, uint32_t directRefs = 0,
+                                            int row0 = 0, int row1 = kTileSize) {
     const uint32_t workItem = kDirect ? workIndex : __builtin_amdgcn_readfirstlane(B.work[workIndex]);
     // segFlag: the segment index, with kSingleSegment >> kTileBits above it
     const uint32_t gtile = workItem & (kMaxBatchTiles - 1), segFlag = workItem >> kTileBits;
@@ -1092,6 +1094,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
     const int tx = (int)(tile % P.tiles_x), ty = (int)(tile / P.tiles_x);
     const int tminX = tx * kTileSize, tminY = ty * kTileSize;
     const int tmaxX = min(tminX + kTileSize, (int)P.width), tmaxY = min(tminY + kTileSize, (int)P.height);
+    const int wminY = kDirect ? tminY + row0 : tminY, wmaxY = kDirect ? min(tminY + row1, tmaxY) : tmaxY;
     const uint32_t start = kDirect ? gtile * B.direct : B.tile_start[gtile];
     const uint32_t n = kDirect ? directRefs : B.tile_start[gtile + 1] - start;
     const uint32_t tileItem = kDirect ? 0u : B.tile_item[gtile], segLog2 = tileItem >> kImageBits;
@@ -1105,7 +1108,9 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
         const SamplePass sp = kMS ? sample_pass(P.sample_level, pass * kPassSamples,
                                                 min(S - pass * kPassSamples, kPassSamples))
                                   : SamplePass{1u, 0u};
-        for (uint32_t i = threadIdx.x; i < sp.n * kKeyPlane<kMS>; i += kThreads) keys[i] = bg_key();
+        for (uint32_t i = threadIdx.x + (kDirect ? row0 * kKeyStride<kMS> : 0);
+             i < (kDirect ? row1 * kKeyStride<kMS> : sp.n * kKeyPlane<kMS>); i += kThreads)
+            keys[i] = bg_key();
         if (!kDirect && threadIdx.x == 0) wide->n = 0;
         __syncthreads();
 
@@ -1140,8 +1145,8 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
             const int by0 = min(t.y0, min(t.y1, t.y2)) >> 4, by1 = max(t.y0, max(t.y1, t.y2)) >> 4;
             minX = max(tminX, bx0);
             maxX = min(tmaxX - 1, bx1);
-            minY = max(tminY, by0);
-            maxY = min(tmaxY - 1, by1);
+            minY = max(wminY, by0);
+            maxY = min(wmaxY - 1, by1);
             return bx1 - bx0 <= 1 && by1 - by0 <= 1;
         };
         // Quads of a reference beyond the tiny path: the first one's pixel, quads per row.
@@ -1199,7 +1204,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
                 const bool isWide = large || myQ >= kWaveQuads || (myQ && !fits);
                 if (kDirect) {
                     walk_wide<kMS>(P, t, pay, large, isWide ? myQ : 0u, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY,
-                                   keys, sp);
+                                   keys, sp, row0 / 8, row1 / 8);
                 } else if (const uint64_t wm = __ballot(isWide)) {
                     uint32_t at = 0;
                     if (lane == 0) at = atomicAdd(&wide->n, (uint32_t)__popcll(wm));
@@ -1308,10 +1313,11 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
 
 // Cleared pixels of an empty tile (as k_shade writes uncovered ones): four pixels
 // per store where the rows start on 16 bytes, else one.  thread: of kThreads that
-// share the tile.
+// share the tile's rows [row0, row1).
 template <uint32_t kThreads>
 __device__ __forceinline__ void clear_tile(const BatchParams& Q, const FrameParams* __restrict__ jobs,
-                                           const DeviceBuffers& B, uint32_t gtile, uint32_t thread) {
+                                           const DeviceBuffers& B, uint32_t gtile, uint32_t thread,
+                                           uint32_t row0 = 0, uint32_t row1 = kTileSize) {
     const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];
     const uint32_t tile = gtile - P.tile_base;
     const int tminX = (int)(tile % P.tiles_x) * kTileSize, tminY = (int)(tile / P.tiles_x) * kTileSize;
@@ -1319,7 +1325,7 @@ __device__ __forceinline__ void clear_tile(const BatchParams& Q, const FramePara
                            4ull * (P.pix_base | P.width);
     if (!(align & 15u)) {
         constexpr uint32_t kRow = kTileSize / 4;
-        for (uint32_t i = thread; i < kRow * kTileSize; i += kThreads) {
+        for (uint32_t i = thread + kRow * row0; i < kRow * row1; i += kThreads) {
             const int x = tminX + (int)(i % kRow) * 4, y = tminY + (int)(i / kRow);
             if (x < (int)P.width && y < (int)P.height) {
                 const size_t o = P.pix_base + (size_t)(P.height - 1 - y) * P.width + x;
@@ -1333,7 +1339,7 @@ __device__ __forceinline__ void clear_tile(const BatchParams& Q, const FramePara
         }
         return;
     }
-    for (uint32_t i = thread; i < kTileSize * kTileSize; i += kThreads) {
+    for (uint32_t i = thread + kTileSize * row0; i < kTileSize * row1; i += kThreads) {
         const int x = tminX + (int)(i % kTileSize), y = tminY + (int)(i / kTileSize);
         if (x < (int)P.width && y < (int)P.height) {
             const size_t o = P.pix_base + (size_t)(P.height - 1 - y) * P.width + x;

@@ -8,6 +8,16 @@ namespace edxr {
 
 namespace {
 constexpr uint32_t kTileThreads = 512;  // k_tile's workgroup
+// Frames of at most this many tiles give a tile two workgroups of 16 rows: where
+// few tiles leave most of the chip idle, a tile's own chain of walks and gathers is
+// k_tile's time.  One and two workgroups: 80 tiles (heightfield at 320x200) 21.4 and
+// 17.4 us, 300 (heightfield, sphere at 640x480) 17.9 and 14.2, 15.5 and 13.2, 475
+// (grid, heightfield at 800x600) 30.9 and 24.1, 19.6 and 16.8, 12 jobs at 256^2 17.8
+// and 13.5; 704 (heightfield, textured at 1000x700) 20.3 and 21.0, 43.5 and 44.4;
+// 2,040 (textured at 1080p) 84 and 88: each workgroup sets up all of the tile's
+// references.  (One workgroup of 1,024 threads: 21.4 and 17.1 us for 80 tiles, but
+// 19.6 and 23.6 for the 475 of the heightfield.)
+constexpr uint32_t kTileHalves = 512;
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -181,9 +191,9 @@ __global__ __launch_bounds__(kBlock) void k_front(BatchParams Q, const FramePara
                           [&](uint32_t tile, int, int, uint32_t payload) { place(tile, payload); });
 }
 
-// One workgroup per tile: rasterises its list and shades the winners from the
-// keys in LDS.
-template <bool kTex>
+// One workgroup per tile, or two of 16 rows each (kHalves): rasterises its list
+// and shades the winners from the keys in LDS.
+template <bool kTex, bool kHalves>
 __global__ __launch_bounds__(kTileThreads, kTex ? 4 : 6) void k_tile(BatchParams Q, const FrameParams* __restrict__ jobs,
                                                                DeviceBuffers B) {
     __shared__ uint64_t keys[kKeyPlane<false>];
@@ -196,24 +206,33 @@ __global__ __launch_bounds__(kTileThreads, kTex ? 4 : 6) void k_tile(BatchParams
             B.counters[i] = 0;
         }
     }
-    const uint32_t gtile = blockIdx.x;
+    const uint32_t gtile = kHalves ? blockIdx.x >> 1 : blockIdx.x;
+    const int row0 = kHalves ? (int)(blockIdx.x & 1u) * (kTileSize / 2) : 0;
+    const int row1 = kHalves ? row0 + kTileSize / 2 : kTileSize;
     if (threadIdx.x == 0) {
-        sCount = min((uint32_t)B.tile_count[gtile], B.direct);
-        B.tile_count[gtile] = 0;
-        B.tile_start[gtile] = sCount;  // (read by edxr_debug_read_bins only)
+        // Of two workgroups the second to read the count word clears it.
+        constexpr uint64_t kRead = 1ull << 63;
+        uint64_t count = kRead;
+        if (kHalves) count = atomicAdd((unsigned long long*)&B.tile_count[gtile], (unsigned long long)kRead);
+        else count |= B.tile_count[gtile];
+        sCount = min((uint32_t)count, B.direct);
+        if (count & kRead) {
+            B.tile_count[gtile] = 0;
+            B.tile_start[gtile] = sCount;  // (read by edxr_debug_read_bins only)
+        }
     }
     __syncthreads();
     const uint32_t n = __builtin_amdgcn_readfirstlane(sCount);
     if (!n) {
-        clear_tile<kTileThreads>(Q, jobs, B, gtile, threadIdx.x);
+        clear_tile<kTileThreads>(Q, jobs, B, gtile, threadIdx.x, row0, row1);
         return;
     }
     const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];
     const uint32_t tile = gtile - P.tile_base;
     const int tminX = (int)(tile % P.tiles_x) * kTileSize, tminY = (int)(tile / P.tiles_x) * kTileSize;
     const int tmaxX = min(tminX + kTileSize, (int)P.width), tmaxY = min(tminY + kTileSize, (int)P.height);
-    raster_item<false, kTileThreads, true>(Q, jobs, B, gtile, keys, sOwner, nullptr, n);
-    for (uint32_t i = threadIdx.x; i < kTileSize * kTileSize; i += kTileThreads) {
+    raster_item<false, kTileThreads, true>(Q, jobs, B, gtile, keys, sOwner, nullptr, n, row0, row1);
+    for (uint32_t i = threadIdx.x + row0 * kTileSize; i < (uint32_t)row1 * kTileSize; i += kTileThreads) {
         const int x = tminX + (int)(i % kTileSize), y = tminY + (int)(i / kTileSize);
         if (x >= tmaxX || y >= tmaxY) continue;
         const uint64_t key = keys[(i / kTileSize) * kKeyStride<false> + i % kTileSize];
@@ -240,9 +259,16 @@ void launch_front(const BatchParams& Q, FrameParams* jobs, const FrameParams* jo
 }
 
 void launch_tile(const BatchParams& Q, const FrameParams* jobs, const DeviceBuffers& B, hipStream_t s) {
-    const dim3 grid(Q.total_tiles);
-    if (Q.any_textured) hipLaunchKernelGGL(k_tile<true>, grid, dim3(kTileThreads), 0, s, Q, jobs, B);
-    else hipLaunchKernelGGL(k_tile<false>, grid, dim3(kTileThreads), 0, s, Q, jobs, B);
+    const bool halves = Q.total_tiles <= kTileHalves;
+    const dim3 grid(halves ? 2 * Q.total_tiles : Q.total_tiles), block(kTileThreads);
+    if (Q.any_textured) {
+        if (halves) hipLaunchKernelGGL((k_tile<true, true>), grid, block, 0, s, Q, jobs, B);
+        else hipLaunchKernelGGL((k_tile<true, false>), grid, block, 0, s, Q, jobs, B);
+    } else if (halves) {
+        hipLaunchKernelGGL((k_tile<false, true>), grid, block, 0, s, Q, jobs, B);
+    } else {
+        hipLaunchKernelGGL((k_tile<false, false>), grid, block, 0, s, Q, jobs, B);
+    }
 }
 
 }  // namespace edxr
