@@ -1436,26 +1436,25 @@ __device__ __forceinline__ uint64_t tile_key(const uint64_t* g, uint32_t nseg, u
 }
 }  // namespace
 
-// One pixel (number pix of the tile) of a single-sample frame's nonempty tile.
+// Low word of the winner's key of a pixel (number pix of the tile) of a
+// single-sample frame's nonempty tile.
+__device__ __forceinline__ uint32_t tile_low(const DeviceBuffers& B, uint32_t tileItem, uint32_t n, uint32_t pix) {
+    constexpr uint32_t kPix = kTileSize * kTileSize;
+    const uint32_t nseg = tile_segments(n, tileItem >> kImageBits);
+    const uint64_t* g = B.partials + (size_t)(tileItem & kImageMask) * kPix;
+    // A single-segment tile's image holds 32-bit low words (k_raster).
+    if (nseg == 1) return reinterpret_cast<const uint32_t*>(g)[pix];
+    const uint64_t key = tile_key(g + pix, nseg, 1, 0);
+    return key == bg_key() ? 0xFFFFFFFFu : (uint32_t)key;
+}
+// That pixel's colour, depth and ID.
 template <bool kTex>
 __device__ __forceinline__ void shade_pixel_of(const FrameParams& P, const DeviceBuffers& B, uint32_t gtile, uint32_t n,
-                                               uint32_t pix) {
-    constexpr uint32_t kPix = kTileSize * kTileSize;
+                                               uint32_t pix, uint32_t low) {
     const uint32_t tile = gtile - P.tile_base;
     const int x = (int)(tile % P.tiles_x) * kTileSize + (int)(pix & 31u);
     const int y = (int)(tile / P.tiles_x) * kTileSize + (int)(pix >> 5);
     if (x >= (int)P.width || y >= (int)P.height) return;
-    const uint32_t tileItem = B.tile_item[gtile];
-    const uint32_t nseg = tile_segments(n, tileItem >> kImageBits);
-    const uint64_t* g = B.partials + (size_t)(tileItem & kImageMask) * kPix;
-    // A single-segment tile's image holds 32-bit low words (k_raster).
-    uint32_t low;
-    if (nseg == 1) {
-        low = reinterpret_cast<const uint32_t*>(g)[pix];
-    } else {
-        const uint64_t key = tile_key(g + pix, nseg, 1, 0);
-        low = key == bg_key() ? 0xFFFFFFFFu : (uint32_t)key;
-    }
     shade_winner<kTex>(P, B, x, y, P.pix_base + (size_t)(P.height - 1 - y) * P.width + x, low,
                        n >= kShadeRecomputeRefs);
 }
@@ -1470,31 +1469,41 @@ __device__ __forceinline__ void shade_tiles(const BatchParams& Q, const FramePar
     const uint32_t gtile = blockIdx.x >> 1;
     const uint32_t n = B.tile_start[gtile + 1] - B.tile_start[gtile];
     if (n == 0) return;
-    shade_pixel_of<kTex>(jobs[job_of(Q, Q.tile_job, gtile)], B, gtile, n,
-                         threadIdx.x + (blockIdx.x & 1u) * kShadeThreads);
+    const uint32_t pix = threadIdx.x + (blockIdx.x & 1u) * kShadeThreads;
+    shade_pixel_of<kTex>(jobs[job_of(Q, Q.tile_job, gtile)], B, gtile, n, pix, tile_low(B, B.tile_item[gtile], n, pix));
 }
 
-// More tiles (batches): the grid's waves take the 16 row pairs of every tile of
-// the work list in turn (a tile's item of segment 0 stands for it), so that no
-// wave is started for an empty tile.  Of the 1.9M waves of two workgroups per
-// tile for 256 jobs three quarters only found their tile empty: 577 us, so 416;
-// 64 views 126 and 81 us.  Where most tiles are covered the list is one load
-// more per tile: 2M sphere grid at 1080p 17 and 20 us, 10M heightfield at 4K 77
-// and 79 us.
+// More tiles (batches): the grid's waves take the tiles of the work list (a tile's
+// item of segment 0 stands for it) in turn, kShadePairs of a tile's 16 row pairs
+// at a time, so that no wave is started for an empty tile.  Of the 1.9M waves of two
+// workgroups per tile for 256 jobs three quarters only found their tile empty: 577
+// us, with a row pair at a time 416, now 404 after a raster that then took 630 us
+// and 450 and 404 after the present one (64 views 126, 78 and 72).  Each step waits
+// on the chain item -> tile -> job -> key image before the gathers: the next item is
+// loaded ahead (409 and 404 us), and four row pairs share a chain (1, 2, 4, 8: 448,
+// 416, 408, 407 us, 64 views 78, 74, 72, 81).  The next pair's key words loaded ahead
+// as well cost more than they hid (408 us).
+constexpr uint32_t kShadePairs = 4;
 template <bool kTex>
 __device__ __forceinline__ void shade_list(const BatchParams& Q, const FrameParams* __restrict__ jobs,
                                            const DeviceBuffers& B) {
-    constexpr uint32_t kPairs = kTileSize * kTileSize / kWave;
+    constexpr uint32_t kUnits = kTileSize * kTileSize / kWave / kShadePairs;
     if (B.counters[kCntOverflow] & kOvNoLists) return;
     const uint32_t waves = gridDim.x * (kShadeThreads / kWave);
-    const uint32_t units = B.counters[kCntWorkItems] * kPairs;
-    for (uint32_t u = __builtin_amdgcn_readfirstlane(blockIdx.x * (kShadeThreads / kWave) + threadIdx.x / kWave);
-         u < units; u += waves) {
-        const uint32_t item = __builtin_amdgcn_readfirstlane(B.work[u / kPairs]);
+    const uint32_t units = B.counters[kCntWorkItems] * kUnits;
+    uint32_t u = __builtin_amdgcn_readfirstlane(blockIdx.x * (kShadeThreads / kWave) + threadIdx.x / kWave);
+    uint32_t nextItem = u < units ? B.work[u / kUnits] : 0u;
+    for (; u < units; u += waves) {
+        const uint32_t item = __builtin_amdgcn_readfirstlane(nextItem);
+        if (u + waves < units) nextItem = B.work[(u + waves) / kUnits];
         if ((item >> kTileBits) & ((1u << kSegIndexBits) - 1)) continue;  // a further segment
         const uint32_t gtile = item & (kMaxBatchTiles - 1);
-        const uint32_t n = B.tile_start[gtile + 1] - B.tile_start[gtile];
-        shade_pixel_of<kTex>(jobs[job_of(Q, Q.tile_job, gtile)], B, gtile, n, (u % kPairs) * kWave + __lane_id());
+        const uint32_t n = B.tile_start[gtile + 1] - B.tile_start[gtile], tileItem = B.tile_item[gtile];
+        const FrameParams& P = jobs[job_of(Q, Q.tile_job, gtile)];
+        uint32_t pix = (u % kUnits) * kShadePairs * kWave + __lane_id();
+#pragma unroll 1
+        for (uint32_t k = 0; k < kShadePairs; k++, pix += kWave)
+            shade_pixel_of<kTex>(P, B, gtile, n, pix, tile_low(B, tileItem, n, pix));
     }
 }
 
