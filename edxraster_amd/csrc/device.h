@@ -1059,14 +1059,21 @@ __device__ __forceinline__ void walk_wide(const FrameParams& P, const RTri& t, u
 
 // An item's references that take a whole wave (tile-level ones, and those of
 // kWaveQuads quads or more), by their place in the item: listed while the
-// slices are walked, kWideRefs of them at most at a time, then shared out over
-// the workgroup's waves.  (Not in a direct frame's tiles: few references, spread
+// slices are walked, then shared out over the workgroup's waves.  At one sample,
+// what the list does not hold any more is walked at once by the wave that has it;
+// places from limit on are not written.  (With the list emptied by all waves
+// after every 1,024 references, so that it never is full, the waves waited for each
+// other: 10M heightfield at 4K k_raster 113 us, so 107, 4.6M triangles on 252 tiles
+// 41 and 37.)  With more samples it is emptied so, after every 512: the second copy
+// of the walk costs that kernel more than the waiting (2.1M sphere grid at 1080p,
+// 4 samples, a call 218 us, 224 with it).
+// (Not in a direct frame's tiles: few references, spread
 // thinly over the waves anyway, whose records would be loaded twice.)
 template <bool kMS>
-constexpr uint32_t kWideRefs = kMS ? 512 : 1024;  // (a multiple of every workgroup's threads)
+constexpr uint32_t kWideRefs = kMS ? 512 : 1024;  // (512: a multiple of the workgroup's threads)
 template <bool kMS>
 struct WideRefs {
-    uint32_t n;
+    uint32_t n, limit;
     uint16_t at[kWideRefs<kMS>];
 };
 
@@ -1111,7 +1118,10 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
         for (uint32_t i = threadIdx.x + (kDirect ? row0 * kKeyStride<kMS> : 0);
              i < (kDirect ? row1 * kKeyStride<kMS> : sp.n * kKeyPlane<kMS>); i += kThreads)
             keys[i] = bg_key();
-        if (!kDirect && threadIdx.x == 0) wide->n = 0;
+        if (!kDirect && threadIdx.x == 0) {
+            wide->n = 0;
+            wide->limit = kWideRefs<kMS>;
+        }
         __syncthreads();
 
         // Each wave takes slices of L references (64, or a quarter of a short
@@ -1160,7 +1170,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
             return (uint32_t)fnx * ((uint32_t)(maxY - minY) / 2u + 1u);
         };
         uint32_t b = segBegin + wave * L;
-        for (uint32_t until = kDirect ? segEnd : segBegin + kWideRefs<kMS>;; until += kWideRefs<kMS>) {
+        for (uint32_t until = kMS ? segBegin + kWideRefs<kMS> : segEnd;; until += kWideRefs<kMS>) {
             for (; b < min(segEnd, until); b += stride) {
                 const uint32_t p = b + lane;
                 const bool valid = lane < L && p < segEnd;
@@ -1202,15 +1212,23 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
                     }
                 }
                 const bool isWide = large || myQ >= kWaveQuads || (myQ && !fits);
-                if (kDirect) {
+                bool walkNow = kDirect;
+                if (!kDirect)
+                    if (const uint64_t wm = __ballot(isWide)) {
+                        const uint32_t count = (uint32_t)__popcll(wm);
+                        uint32_t at = 0;
+                        if (lane == 0) at = atomicAdd(&wide->n, count);
+                        at = __builtin_amdgcn_readfirstlane(at);
+                        walkNow = !kMS && at + count > kWideRefs<kMS>;
+                        if (walkNow) {
+                            if (lane == 0) atomicMin(&wide->limit, at);
+                        } else if (isWide) {
+                            wide->at[at + (uint32_t)__popcll(wm & lanemask_lt())] = (uint16_t)(p - segBegin);
+                        }
+                    }
+                if (walkNow)
                     walk_wide<kMS>(P, t, pay, large, isWide ? myQ : 0u, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY,
                                    keys, sp, row0 / 8, row1 / 8);
-                } else if (const uint64_t wm = __ballot(isWide)) {
-                    uint32_t at = 0;
-                    if (lane == 0) at = atomicAdd(&wide->n, (uint32_t)__popcll(wm));
-                    at = __builtin_amdgcn_readfirstlane(at);
-                    if (isWide) wide->at[at + (uint32_t)__popcll(wm & lanemask_lt())] = (uint16_t)(p - segBegin);
-                }
                 if (isWide) myQ = 0;
                 // Other references with quads: the wave's quads are expanded into
                 // (reference, quad) pairs and tested 64 per pass, one quad per lane.
@@ -1267,7 +1285,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
             // 127 with 4 samples; so 36 and 86.  With a quadrant or 64 quads of each
             // reference per wave its preparation by four waves cost more than the
             // finer split gave: 40 and 86.)
-            const uint32_t nWide = __builtin_amdgcn_readfirstlane(wide->n);
+            const uint32_t nWide = __builtin_amdgcn_readfirstlane(min(wide->n, wide->limit));
             for (uint32_t e0 = 0; e0 < nWide; e0 += kThreads) {
                 const uint32_t e = e0 + wave + kThreads / kWave * lane;
                 const bool valid = e < nWide;
