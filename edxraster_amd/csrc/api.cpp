@@ -1690,9 +1690,9 @@ int64_t edxr_debug_read_bins(edxr_ctx* c, uint64_t* offsets, uint32_t* refs3, ui
     if (refs3 && total <= cap) {
         for (uint64_t i = 0; i < total; i++) {
             const uint32_t p = refs[i], ri = p & kRecordMask;
-            const uint32_t acc = (p >> kRecordBits) & 7u;
             const uint32_t big = p >> 31;
-            const bool compact = !big && ri < c->lastT;  // record slot = triangle, not stored
+            const uint32_t acc = big ? (p >> kRecordBits) & 7u : 0u;
+            const bool compact = p <= kRecordMask;  // record slot = triangle, not stored
             refs3[3 * i] = compact ? ri : rr[ri].order >> 4;
             refs3[3 * i + 1] = compact ? 0u : (rr[ri].info >> 12) & 7u;
             refs3[3 * i + 2] = acc | ((acc == 7u) ? 8u : 0u) | (big ? 16u : 0u);

@@ -372,6 +372,18 @@ __device__ __forceinline__ int any_non_compact(const uint32_t (&d)[kN]) {
     return any ? 1 : 0;
 }
 
+// Whether a reference counts as a heavy one of its tile.
+__device__ __forceinline__ bool heavy_ref(uint32_t payload) {
+    return payload >> 31 || (payload & (kRefStored | kRefHeavy)) == (kRefStored | kRefHeavy);
+}
+// The reference of record rec in a tile that its small box lists untested.
+__device__ __forceinline__ uint32_t small_ref(const BinTri& b, uint32_t rec) {
+    const uint32_t ex = (uint32_t)max(b.x0, max(b.x1, b.x2)) - (uint32_t)min(b.x0, min(b.x1, b.x2));
+    const uint32_t ey = (uint32_t)max(b.y0, max(b.y1, b.y2)) - (uint32_t)min(b.y0, min(b.y1, b.y2));
+    const bool heavy = max(ex, ey) >= kCompactExtent && (uint64_t)(ex >> 4) * (ey >> 4) >= kHeavyPixels;
+    return rec | kRefStored | (heavy ? kRefHeavy : 0u);
+}
+
 // The references of record rec (its tile bbox loaded in b) whose bbox tiles
 // are k0, k0 + dk, ... (row-major over the bbox), passed to emit(tile, tx,
 // ty, payload).
@@ -388,7 +400,7 @@ __device__ __forceinline__ void enum_record_tiles(const FrameParams& P, const Bi
         const int f = b.small ? 0 : bin_test(b, tx, ty);
         if (f >= 0)
             emit((uint32_t)ty * P.tiles_x + (uint32_t)tx, tx, ty,
-                 b.small ? rec : rec | ((uint32_t)f << kRecordBits) | (1u << 31));
+                 b.small ? small_ref(b, rec) : rec | ((uint32_t)f << kRecordBits) | (1u << 31));
         cx += dx;
         cy += dy;
         if (cx >= w) {
@@ -1178,7 +1190,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
                 const uint32_t rid = pay & kRecordMask;
                 const bool trivial = ((pay >> kRecordBits) & 7u) == 7u;
                 const bool big = (pay >> 31) != 0;
-                const bool compact = !big && rid < Q.total_slots;
+                const bool compact = pay <= kRecordMask;
                 const ScreenVert s0 = n0, s1 = n1, s2 = n2;
                 sv_of(idx2, n0, n1, n2);
                 idx2 = ref_indices(P, pay3);
@@ -1294,7 +1306,7 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
                 const bool big = (pay >> 31) != 0, trivial = ((pay >> kRecordBits) & 7u) == 7u;
                 const bool large = valid && (trivial || (big && P.hierarchical));
                 RTri t;
-                if (big || rid >= Q.total_slots) load_rtri(B.rrec[rid], t);
+                if (pay > kRecordMask) load_rtri(B.rrec[rid], t);
                 else screen_rtri(P, B, rid, t);
                 uint32_t quads = 0;
                 int fx = 0, fy = 0, fnx = 1;

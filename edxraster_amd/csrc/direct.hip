@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kBlock) void k_front(BatchParams Q, const FramePara
     if (nBig)
         block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
                           [&](uint32_t tile, int tx, int ty, uint32_t payload) {
-                              atomicAdd(&hist[tile], payload >> 31 ? 0x10001u : 1u);
+                              atomicAdd(&hist[tile], heavy_ref(payload) ? 0x10001u : 1u);
                               bx0 = min(bx0, (uint32_t)tx);
                               by0 = min(by0, (uint32_t)ty);
                               bx1 = max(bx1, (uint32_t)tx);

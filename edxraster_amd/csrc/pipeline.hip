@@ -542,7 +542,7 @@ __global__ __launch_bounds__(kClipWaves * 64) void k_clip(BatchParams Q, const F
                     const uint32_t rec = first + (uint32_t)__popcll(fanMask & ((1ull << l) - 1ull));
                     enum_record_tiles(P, bt, rec, lane, kWave, [&](uint32_t tile, int, int, uint32_t payload) {
                         const uint32_t g = P.tile_base + tile;
-                        const uint64_t one = payload >> 31 ? 1ull << 32 | 1ull : 1ull;
+                        const uint64_t one = heavy_ref(payload) ? 1ull << 32 | 1ull : 1ull;
                         const uint64_t old = atomicAdd((unsigned long long*)&B.tile_count[g], (unsigned long long)one);
                         direct_check(B, old + one);
                         refs++;
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_count(BatchParams Q, const Frame
             __syncthreads();
             block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
                               [&](uint32_t tile, int tx, int ty, uint32_t payload) {
-                                  bump(tile, (payload >> 31) != 0);
+                                  bump(tile, heavy_ref(payload));
                                   bx0 = min(bx0, (uint32_t)tx);
                                   by0 = min(by0, (uint32_t)ty);
                                   bx1 = max(bx1, (uint32_t)tx);
