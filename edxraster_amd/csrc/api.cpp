@@ -425,7 +425,10 @@ int build_plan(edxr_ctx* c, const std::vector<JobInput>& in, Plan& pl) {
         Q.max_job_tiles = std::max(Q.max_job_tiles, P.num_tiles);
         Q.max_job_chunks = std::max(Q.max_job_chunks, P.num_chunks);
         Q.max_samples = std::max(Q.max_samples, P.samples);
-        if (P.shader == kTexturedLambert) Q.any_textured = 1;
+        if (P.shader == kTexturedLambert) {
+            Q.any_textured = 1;
+            if (P.tex_filter >= kFilterAniso4) Q.any_aniso = 1;
+        }
         pl.jobs.push_back(P);
         if (vert > 0xF0000000ull || slot + 65536 > kRecordMask) return c->fail(EDXR_E_LIMIT, "too many triangles");
     }

@@ -150,6 +150,7 @@ struct BatchParams {
     uint32_t max_job_chunks;    // max over jobs of num_chunks
     uint32_t max_samples;       // max over jobs of samples
     uint32_t any_textured;      // 1 if a job uses the textured shader
+    uint32_t any_aniso;         // 1 if one of those filters anisotropically
     const uint32_t* vblock_job;
     const uint32_t* sblock_job;
     const uint32_t* chunk_job;

@@ -1459,9 +1459,10 @@ __device__ __forceinline__ void shade_pixel_of(const FrameParams& P, const Devic
                        n >= kShadeRecomputeRefs);
 }
 
-// Single-sample frames of up to kShadeListTiles tiles: two workgroups per tile,
-// 16 rows each (smaller workgroups than one per tile schedule better and cost
-// less where the tile is empty, cleared by k_raster).
+// Single-sample frames of up to kShadeListTiles tiles, and larger ones of one job
+// with an anisotropic filter: two workgroups per tile, 16 rows each (smaller
+// workgroups than one per tile schedule better and cost less where the tile is
+// empty, cleared by k_raster).
 template <bool kTex>
 __device__ __forceinline__ void shade_tiles(const BatchParams& Q, const FrameParams* __restrict__ jobs,
                                             const DeviceBuffers& B) {
@@ -1483,6 +1484,13 @@ __device__ __forceinline__ void shade_tiles(const BatchParams& Q, const FramePar
 // loaded ahead (409 and 404 us), and four row pairs share a chain (1, 2, 4, 8: 448,
 // 416, 408, 407 us, 64 views 78, 74, 72, 81).  The next pair's key words loaded ahead
 // as well cost more than they hid (408 us).
+// Calls with two workgroups per tile and so: 64 spheres at 512^2 (a third of the
+// tiles covered) 419 and 334 us textured, 868 and 625 anisotropic; 9 covered jobs at
+// 1024^2 380 and 365, 478 and 454, 795 and 808; 17 at 1080p 923 and 933.  One frame of
+// 16,384 tiles: sphere 331 and 324, covered heightfield of 2M triangles 539 and 536,
+// trilinear 743 and 740, but 1,467 and 1,710 at 8:1 (a pixel's taps are then the
+// work, and a wave's four row pairs end the pass); of 9,216 444 and 445; of 8,448 190
+// and 193.
 constexpr uint32_t kShadePairs = 4;
 template <bool kTex>
 __device__ __forceinline__ void shade_list(const BatchParams& Q, const FrameParams* __restrict__ jobs,
@@ -1746,7 +1754,7 @@ hipError_t launch_frame(const BatchParams& Q, FrameParams* jobs, const FramePara
         else hipLaunchKernelGGL(plain, grid, shadeThreads, 0, s, Q, jobs, B);
     };
     if (Q.max_samples > 1) shade(k_shade<kShadeSamples>, k_shade_tex<kShadeSamples>, dim3(2 * Q.total_tiles));
-    else if (Q.total_tiles > kShadeListTiles)
+    else if (Q.total_tiles > kShadeListTiles && (Q.num_jobs > 1 || !Q.any_aniso))
         shade(k_shade<kShadeList>, k_shade_tex<kShadeList>, dim3(kShadeGroups * B.num_cus));
     else shade(k_shade<kShadeTiles>, k_shade_tex<kShadeTiles>, dim3(2 * Q.total_tiles));
     mark(5);
