@@ -473,8 +473,9 @@ void drop_graph(edxr_ctx* c) {
 // average for spheres, 2 to 5 times for sphere grids and 6 to 12 times for
 // heightfields, from 320x200 to 1080p; such a frame pays for both paths and
 // their buffers (first frame of a context 416 us general alone, 636 with both).
-// Not with capacities or chunks set by the caller, which are the general
-// path's.
+// Not with capacities or bin chunks set by the caller, which are the general
+// path's.  (Triangles per chunk and raster blocks per CU, set or tuned, only steer
+// that path where it is taken.)
 bool direct_frame(edxr_ctx* c, const BatchParams& Q) {
     if (Q.max_samples != 1 || !Q.total_slots || Q.total_tiles > kDirectMaxTiles ||
         Q.total_slots > kDirectMaxSlots || c->debugCapacity || (Q.num_jobs == 1 && c->binChunksSetting) ||
@@ -1483,32 +1484,49 @@ int edxr_autotune(edxr_ctx* c, const edxr_job* jobs, uint32_t n, edxr_tuning* ou
     static const uint32_t kTpc[] = {512, 1024, 2048, 4096};
     static const uint32_t kRpc[] = {4, 8, 16};
     const uint32_t saveT = c->trisPerChunk, saveR = c->rasterPerCU;
+    double ms = 0.0;
+    // The median of seven frames (candidates often differ by 1-2 %), after one
+    // that allocates and captures.
+    auto frames = [&](bool first) {
+        int r = first ? edxr_render_batch(c, jobs, n) : EDXR_OK;
+        double times[7];
+        for (double& t : times) {
+            const auto t0 = std::chrono::steady_clock::now();
+            if (r == EDXR_OK) r = edxr_render_batch(c, jobs, n);
+            t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        }
+        std::sort(times, times + 7);
+        ms = times[3];
+        return r;
+    };
+    // Direct frames have neither chunks nor segments: jobs that take them leave
+    // the settings as they are (the candidates would differ by noise only, and the
+    // chosen one would steer the context's later general frames).
+    c->directSkip = 0;
+    int r = edxr_render_batch(c, jobs, n);
+    if (r != EDXR_OK) return r;
+    if (c->lastDirect) {
+        if ((r = frames(false)) != EDXR_OK) return r;
+        if (out) {
+            out->tris_per_chunk = saveT ? saveT : 1024;
+            out->raster_blocks_per_cu = saveR ? saveR : 8;
+            out->frame_ms = ms;
+        }
+        return EDXR_OK;
+    }
     double best = 1e30;
     uint32_t bestT = 1024, bestR = 8;
     for (uint32_t tpc : kTpc)
         for (uint32_t rpc : kRpc) {
             c->trisPerChunk = tpc;
             c->rasterPerCU = rpc;
-            int r = edxr_render_batch(c, jobs, n);  // warm-up (allocation, capture)
-            if (r != EDXR_OK) {
+            if ((r = frames(true)) != EDXR_OK) {
                 c->trisPerChunk = saveT;
                 c->rasterPerCU = saveR;
                 return r;
             }
-            // the median of seven frames: candidates often differ by 1-2 %
-            double times[7];
-            for (double& t : times) {
-                const auto t0 = std::chrono::steady_clock::now();
-                if ((r = edxr_render_batch(c, jobs, n)) != EDXR_OK) {
-                    c->trisPerChunk = saveT;
-                    c->rasterPerCU = saveR;
-                    return r;
-                }
-                t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-            }
-            std::sort(times, times + 7);
-            if (times[3] < best) {
-                best = times[3];
+            if (ms < best) {
+                best = ms;
                 bestT = tpc;
                 bestR = rpc;
             }

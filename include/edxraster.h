@@ -98,7 +98,12 @@ enum edxr_state_key {
     /* 1 = capture each frame's launches in a HIP graph and replay it while the
      * launch layout (sizes, capacities, tuning) repeats; default 0. */
     EDXR_STATE_GRAPH = 4,
-    /* Triangles per binning chunk (0 = automatic, 1024). */
+    /* Triangles per binning chunk (0 = automatic: 1024, with at most 2,048
+     * chunks per job of more than 4,096 tiles).  This setting and the next one
+     * steer the general path only: small single-sample frames and batches (up
+     * to 1,048,576 triangle slots, 416 per tile and 32,768 tiles, no bin chunks
+     * set) take a direct path, which lists references per tile without chunks
+     * or segments, unless a tile is too deep for it. */
     EDXR_STATE_TRIS_PER_CHUNK = 5,
     /* Raster work items per compute unit that the tile-segment size aims for
      * (0 = automatic, 8); the raster grid itself is always as many
@@ -301,7 +306,9 @@ int edxr_batch_read(edxr_ctx* ctx, uint32_t job, uint8_t* rgba, float* depth, ui
 int edxr_batch_device_buffers(edxr_ctx* ctx, void** color, void** depth, void** ids, uint64_t* pixel_offsets);
 /* Times candidate (triangles per chunk, raster work items per CU) pairs on the
  * given batch (or single job, num_jobs = 1), keeps the fastest in the
- * context's state and returns it in *out (may be NULL). */
+ * context's state and returns it in *out (may be NULL).  Jobs that take the
+ * direct path (see EDXR_STATE_TRIS_PER_CHUNK), which has neither, leave the
+ * state as it is; *out then holds its values and the present time. */
 int edxr_autotune(edxr_ctx* ctx, const edxr_job* jobs, uint32_t num_jobs, edxr_tuning* out);
 
 /* ---- differentiation (no counterpart in the reference) ---- */
