@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .renderer import Renderer, _check
+from .renderer import Renderer, _check, _mat
 
 
 def _ptr(t):
@@ -64,7 +64,11 @@ def _view_jobs(mesh, views, light, shader, material):
     field("width", [int(v.width) for v in views], np.uint32)
     field("height", [int(v.height) for v in views], np.uint32)
     for name in ("mv", "proj", "raster"):
-        m = np.concatenate([getattr(v, name) for v in views], axis=None)
+        mats = [getattr(v, name) for v in views]
+        try:
+            m = np.asarray(mats, np.float32)  # of one shape
+        except ValueError:
+            m = np.stack([_mat(x) for x in mats])
         if m.size != 16 * len(views):
             raise ValueError("%s must have 16 entries per view" % name)
         field(name, m, np.float32)
