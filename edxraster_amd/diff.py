@@ -46,6 +46,12 @@ def check_inputs(indices, planes):
             raise ValueError("%s must be on the CUDA device of px (got %s)" % (name, t.device))
 
 
+def _floats(t):
+    """The values of t, flat or with further sides of one, as floats."""
+    t = t.detach()
+    return t.tolist() if t.dim() == 1 else [float(x) for x in t.cpu()]
+
+
 def _view_jobs(mesh, views, light, shader, material):
     """edxr_job array of one mesh, light and material seen from `views`: the
     first job is filled by Renderer.make_job and copied for the others, which
@@ -83,7 +89,7 @@ class _RenderViews(torch.autograd.Function):
         idx = indices.contiguous()
         V, T = planes[0].numel(), idx.numel() // 3
         mesh = L.Mesh(*[_ptr(t) for t in planes], C.cast(C.c_void_p(idx.data_ptr()), L.U32), V, T, L.MEM_DEVICE)
-        lt, mt = light.detach().tolist(), material.detach().tolist()
+        lt, mt = _floats(light), _floats(material)
         mat = L.Material()
         mat.ambient, mat.kd, mat.ks, mat.shininess = mt
         mat.albedo[:] = [1.0, 1.0, 1.0]

@@ -1,6 +1,6 @@
 """Jobs of differentiable views, copied from a template: byte for byte those of
 Renderer.make_job for every form of matrix that it takes, and what it refuses is
-refused."""
+refused; and the forms of light and material tensors."""
 import numpy as np
 import pytest
 import torch
@@ -53,3 +53,16 @@ def test_matrices_of_other_sizes_are_refused(built, name, sizes):
         setattr(v, name, np.resize(getattr(v, name), n))
     with pytest.raises(ValueError):
         diff._view_jobs(L.Mesh(), vs, LIGHT, L.SHADER_VC_BLINN_PHONG, material())
+
+
+@pytest.mark.parametrize("shape", [(3,), (3, 1), (3, 1, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16, torch.int32])
+def test_light_and_material_forms(shape, dtype):
+    t = torch.tensor([1.0, -2.0, 3.0]).to(dtype).reshape(shape).requires_grad_(dtype.is_floating_point)
+    assert diff._floats(t) == [1.0, -2.0, 3.0]
+
+
+@pytest.mark.parametrize("shape", [(), (1, 3), (3, 2)])
+def test_other_forms_are_refused(shape):
+    with pytest.raises((TypeError, ValueError, RuntimeError)):
+        diff._floats(torch.ones(shape))
