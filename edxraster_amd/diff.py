@@ -81,6 +81,15 @@ def _view_jobs(mesh, views, light, shader, material):
     return jobs
 
 
+def _split_grads(out, V, device):
+    """The nine planes of out and, on device, the light's and the material's values.
+    (No views of several outputs, and no views of light and material: autograd
+    refuses to let a program change those in place.)"""
+    planes = out[:9 * V].view(9, V)
+    rest = out[9 * V:].to(device)
+    return [planes[k] for k in range(9)] + [rest[:3].clone(), rest[3:].clone()]
+
+
 class _RenderViews(torch.autograd.Function):
     @staticmethod
     def forward(ctx, rend, views, shader, indices, px, py, pz, nx, ny, nz, cr, cg, cb, light, material):
@@ -127,9 +136,7 @@ class _RenderViews(torch.autograd.Function):
         arr = (L.Grads * ctx.njobs)()
         np.frombuffer(arr, np.uint64).reshape(ctx.njobs, 11)[:] = gr
         _check(ctx.rend.ctx, L.lib().edxr_backward(ctx.rend.ctx, _ptr(g), arr, ctx.njobs))
-        gv = out[:9 * ctx.V].view(9, ctx.V).unbind(0)
-        gs = out[9 * ctx.V:].to(ctx.light_device)
-        return (None, None, None, None, *gv, gs[:3], gs[3:])
+        return (None, None, None, None, *_split_grads(out, ctx.V, ctx.light_device))
 
 
 def render_views(rend, views, indices, px, py, pz, nx, ny, nz, cr, cg, cb, light, material,

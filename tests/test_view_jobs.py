@@ -1,6 +1,7 @@
 """Jobs of differentiable views, copied from a template: byte for byte those of
 Renderer.make_job for every form of matrix that it takes, and what it refuses is
-refused; and the forms of light and material tensors."""
+refused; the forms of light and material tensors; and what may be done with the
+gradients."""
 import numpy as np
 import pytest
 import torch
@@ -66,3 +67,25 @@ def test_light_and_material_forms(shape, dtype):
 def test_other_forms_are_refused(shape):
     with pytest.raises((TypeError, ValueError, RuntimeError)):
         diff._floats(torch.ones(shape))
+
+
+class _Gradients(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *inputs):
+        return sum(t.sum() for t in inputs)
+
+    @staticmethod
+    def backward(ctx, g):
+        return tuple(diff._split_grads(torch.arange(9 * 5 + 7.0), 5, "cpu"))
+
+
+@pytest.mark.parametrize("k,create_graph", [(0, True), (8, True), (9, False), (9, True), (10, False), (10, True)])
+def test_gradients_change_in_place(k, create_graph):
+    """With a graph of the gradients any of them, without one the light's and the
+    material's (planes are then views made without one), take values that have a
+    gradient themselves."""
+    inputs = [torch.zeros(n, requires_grad=True) for n in [5] * 9 + [3, 4]]
+    grads = torch.autograd.grad(_Gradients.apply(*inputs), inputs, create_graph=create_graph)
+    assert torch.equal(torch.cat(grads), torch.arange(9 * 5 + 7.0))
+    grads[k].add_(inputs[0].sum())
+    assert grads[k].requires_grad
