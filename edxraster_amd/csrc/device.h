@@ -60,14 +60,14 @@ __device__ __forceinline__ uint32_t clip_code(const float4& v) {
 // reciprocal, and one residual step a correctly rounded quotient or square root
 // (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000
 // processor", 1990): 3 and 3 instructions, not the 10 of a division whose operands
-// may be anything.  Every float of the ranges below gives the bits of 1.0f / x and
-// 1.0f / sqrtf(x), and so did 7e10 pairs those of a / w.  2.1M sphere grid at 1080p,
-// 4 samples: k_shade 47.3 us with divisions, 41.8 so (16 colours of a pixel are
-// divided by 255), a call 217.3 and 215.0; k_tile of 98K triangles 23.6 and 22.2, a
-// call 49.2 and 47.5.  Larger frames are bound by the gathers of vertices: k_shade
-// of the 10M heightfield at 4K 75.0 and 71.8, of 256 jobs 453 and 449, the calls
-// within their spread.  Vertices are transformed with divisions: k_vertex is bound by
-// memory (256 jobs 173 us, 177 so).
+// may be anything.  tests/test_quotients_all.py compares the bits with those of
+// 1.0f / x and 1.0f / sqrtf(x) for every float, and of projections for 2^35 points a
+// seed.  2.1M sphere grid at 1080p, 4 samples: k_shade 47.3 us with divisions, 41.8 so
+// (16 colours of a pixel are divided by 255), a call 217.3 and 215.0; k_tile of 98K
+// triangles 23.6 and 22.2, a call 49.2 and 47.5.  Larger frames are bound by the
+// gathers of vertices: k_shade of the 10M heightfield at 4K 75.0 and 71.8, of 256 jobs
+// 453 and 449, the calls within their spread.  Vertices are transformed with
+// divisions: k_vertex is bound by memory (256 jobs 173 us, 177 so).
 
 // Whether x lies in [2^lo, 2^hi) (not a negative number or NaN).
 template <int kLo, int kHi>
@@ -79,7 +79,9 @@ __device__ __forceinline__ float rcp_normal(float x) {
     const float y = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
 }
-// a / x from y = 1 / x: x in [2^-60, 2^60), |a| in [2^-100, 2^60] or 0 (whose sign is lost).
+// a / x from y = 1 / x: x in [2^-60, 2^60), |a| in [2^-64, 2^60], so that the quotient
+// is a normal number (with |a| from 2^-100 on, one subnormal quotient in some 3e9 pairs came out
+// one step off), or 0 (whose sign is lost).
 __device__ __forceinline__ float quotient_normal(float a, float x, float y) {
     const float q = a * y;
     return __builtin_fmaf(__builtin_fmaf(-x, q, a), y, q);
@@ -99,7 +101,7 @@ __device__ __forceinline__ float reciprocal_sqrt(float x) {
 // A clip-space point's homogeneous projection x / w, y / w, z / w and z * (1 / w).
 // (A projection that only differs in the sign of a zero is the same to snap_point.)
 __device__ __forceinline__ bool project_is_normal(const float4& c) {
-    return in_range<-60, 60>(c.w) && fminf(fminf(fabsf(c.x), fabsf(c.y)), fabsf(c.z)) >= 0x1p-100f &&
+    return in_range<-60, 60>(c.w) && fminf(fminf(fabsf(c.x), fabsf(c.y)), fabsf(c.z)) >= 0x1p-64f &&
            fmaxf(fmaxf(fabsf(c.x), fabsf(c.y)), fabsf(c.z)) <= 0x1p60f;
 }
 __device__ __forceinline__ float4 project_normal(const float4& c) {
