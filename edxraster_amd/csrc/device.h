@@ -374,27 +374,24 @@ __device__ __forceinline__ int any_non_compact(const uint32_t (&d)[kN]) {
     return any ? 1 : 0;
 }
 
-// Whether a reference counts as a heavy one of its tile.
-__device__ __forceinline__ bool heavy_ref(uint32_t payload) {
-    return payload >> 31 || (payload & (kRefStored | kRefHeavy)) == (kRefStored | kRefHeavy);
-}
-// The reference of record rec in a tile that its small box lists untested.
-__device__ __forceinline__ uint32_t small_ref(const BinTri& b, uint32_t rec) {
+// Whether the references of a record whose small box is listed untested count as
+// heavy ones: those of a triangle too long for a compact descriptor, as kDescHeavy.
+__device__ __forceinline__ bool small_heavy(const BinTri& b) {
     const uint32_t ex = (uint32_t)max(b.x0, max(b.x1, b.x2)) - (uint32_t)min(b.x0, min(b.x1, b.x2));
     const uint32_t ey = (uint32_t)max(b.y0, max(b.y1, b.y2)) - (uint32_t)min(b.y0, min(b.y1, b.y2));
-    const bool heavy = max(ex, ey) >= kCompactExtent && (uint64_t)(ex >> 4) * (ey >> 4) >= kHeavyPixels;
-    return rec | kRefStored | (heavy ? kRefHeavy : 0u);
+    return max(ex, ey) >= kCompactExtent && (uint64_t)(ex >> 4) * (ey >> 4) >= kHeavyPixels;
 }
 
 // The references of record rec (its tile bbox loaded in b) whose bbox tiles
 // are k0, k0 + dk, ... (row-major over the bbox), passed to emit(tile, tx,
-// ty, payload).
+// ty, payload, heavy).
 template <class Emit>
 __device__ __forceinline__ void enum_record_tiles(const FrameParams& P, const BinTri& b, uint32_t rec, uint32_t k0,
                                                   uint32_t dk, Emit&& emit) {
     const uint32_t n = (uint32_t)(b.w * b.h);
     if (n == 0) return;
     const uint32_t w = (uint32_t)b.w;
+    const bool heavy = !b.small || small_heavy(b);
     uint32_t cx = k0 % w, cy = k0 / w;
     const uint32_t dx = dk % w, dy = dk / w;
     for (uint32_t k = k0; k < n; k += dk) {
@@ -402,7 +399,7 @@ __device__ __forceinline__ void enum_record_tiles(const FrameParams& P, const Bi
         const int f = b.small ? 0 : bin_test(b, tx, ty);
         if (f >= 0)
             emit((uint32_t)ty * P.tiles_x + (uint32_t)tx, tx, ty,
-                 b.small ? small_ref(b, rec) : rec | ((uint32_t)f << kRecordBits) | (1u << 31));
+                 b.small ? rec | kRefStored : rec | ((uint32_t)f << kRecordBits) | (1u << 31), heavy);
         cx += dx;
         cy += dy;
         if (cx >= w) {

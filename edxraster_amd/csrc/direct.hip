@@ -137,8 +137,8 @@ __global__ __launch_bounds__(kBlock) void k_front(BatchParams Q, const FramePara
     const uint32_t nBig = sBigN;
     if (nBig)
         block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
-                          [&](uint32_t tile, int tx, int ty, uint32_t payload) {
-                              atomicAdd(&hist[tile], heavy_ref(payload) ? 0x10001u : 1u);
+                          [&](uint32_t tile, int tx, int ty, uint32_t, bool heavy) {
+                              atomicAdd(&hist[tile], heavy ? 0x10001u : 1u);
                               bx0 = min(bx0, (uint32_t)tx);
                               by0 = min(by0, (uint32_t)ty);
                               bx1 = max(bx1, (uint32_t)tx);
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kBlock) void k_front(BatchParams Q, const FramePara
     }
     if (nBig)
         block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
-                          [&](uint32_t tile, int, int, uint32_t payload) { place(tile, payload); });
+                          [&](uint32_t tile, int, int, uint32_t payload, bool) { place(tile, payload); });
 }
 
 // One workgroup per tile, or two of 16 rows each (kHalves): rasterises its list

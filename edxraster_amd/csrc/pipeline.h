@@ -72,11 +72,10 @@ constexpr uint32_t kHeavyPixels = 256;
 constexpr uint32_t kCompactExtent = 1u << 14;  // of a compact triangle's bounding box, in 1/16 pixels
 // A tile's reference: a compact triangle's is its slot alone (its screen values
 // are read from the vertices, its products taken in 24 bits); any other has a bit
-// above the record's set, as its record is stored.  A record tested against the
-// tile: bit 31 and the edges that accept the tile in bits 28..30.  One that spans
-// at most 2x2 tiles, listed untested: kRefStored, and kRefHeavy (as kDescHeavy)
-// for a triangle of kCompactExtent or more.
-constexpr uint32_t kRefStored = 1u << kRecordBits, kRefHeavy = 2u << kRecordBits;
+// above the record's set, as its record is stored: bit 31 and the edges that accept
+// the tile in bits 28..30, or, for a record whose box of at most 2x2 tiles is listed
+// untested, kRefStored.
+constexpr uint32_t kRefStored = 1u << kRecordBits;
 
 enum ShaderKind { kLambertAlbedo = 0, kBlinnPhongRef = 1, kVcBlinnPhong = 2, kTexturedLambert = 3 };
 enum TextureFilter {

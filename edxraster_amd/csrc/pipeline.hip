@@ -540,9 +540,9 @@ __global__ __launch_bounds__(kClipWaves * 64) void k_clip(BatchParams Q, const F
                     BinTri bt;
                     load_bin_tri(P, u, bt);
                     const uint32_t rec = first + (uint32_t)__popcll(fanMask & ((1ull << l) - 1ull));
-                    enum_record_tiles(P, bt, rec, lane, kWave, [&](uint32_t tile, int, int, uint32_t payload) {
+                    enum_record_tiles(P, bt, rec, lane, kWave, [&](uint32_t tile, int, int, uint32_t payload, bool heavy) {
                         const uint32_t g = P.tile_base + tile;
-                        const uint64_t one = heavy_ref(payload) ? 1ull << 32 | 1ull : 1ull;
+                        const uint64_t one = heavy ? 1ull << 32 | 1ull : 1ull;
                         const uint64_t old = atomicAdd((unsigned long long*)&B.tile_count[g], (unsigned long long)one);
                         direct_check(B, old + one);
                         refs++;
@@ -634,8 +634,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_count(BatchParams Q, const Frame
             }
             __syncthreads();
             block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
-                              [&](uint32_t tile, int tx, int ty, uint32_t payload) {
-                                  bump(tile, heavy_ref(payload));
+                              [&](uint32_t tile, int tx, int ty, uint32_t, bool heavy) {
+                                  bump(tile, heavy);
                                   bx0 = min(bx0, (uint32_t)tx);
                                   by0 = min(by0, (uint32_t)ty);
                                   bx1 = max(bx1, (uint32_t)tx);
@@ -1329,7 +1329,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_scatter(BatchParams Q, const Fra
             }
             __syncthreads();
             block_enum_listed(P, B.rrec, sBig, nBig, sScan, sWide, &sWideN,
-                              [&](uint32_t tile, int, int, uint32_t payload) {
+                              [&](uint32_t tile, int, int, uint32_t payload, bool) {
                                   B.refs[atomicAdd(&cursor[tile], 1u)] = payload;
                               });
             __syncthreads();  // the lists are rewritten by the next step
