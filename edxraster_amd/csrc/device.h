@@ -1297,8 +1297,16 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
             // reference per wave its preparation by four waves cost more than the
             // finer split gave: 40 and 86.)
             const uint32_t nWide = __builtin_amdgcn_readfirstlane(min(wide->n, wide->limit));
+            // With more samples and fewer references than waves, two or four waves
+            // share each, by quadrants or by rows of quads: large triangles' tiles
+            // have one to four, and one wave of eight walking took longer than of four
+            // (200 triangles on 2454x2310, 4 samples, a call 360 us, so 322; 338 with
+            // workgroups of four waves and none shared).
+            constexpr uint32_t kWaves = kThreads / kWave;
+            const uint32_t parts = !kMS ? 1u : 4 * nWide <= kWaves ? 4u : 2 * nWide <= kWaves ? 2u : 1u;
+            const uint32_t part = wave % parts;
             for (uint32_t e0 = 0; e0 < nWide; e0 += kThreads) {
-                const uint32_t e = e0 + wave + kThreads / kWave * lane;
+                const uint32_t e = e0 + wave / parts + kWaves / parts * lane;
                 const bool valid = e < nWide;
                 const uint32_t pay = segRefs[segBegin + wide->at[valid ? e : 0u]];
                 const uint32_t rid = pay & kRecordMask;
@@ -1313,8 +1321,14 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
                     int minX, maxX, minY, maxY;
                     pixel_box(t, minX, maxX, minY, maxY);
                     quads = quad_box(minX, maxX, minY, maxY, fx, fy, fnx);
+                    if (kMS) {
+                        const uint32_t rows = quads / (uint32_t)fnx, r0 = rows * part / parts;
+                        quads = (rows * (part + 1) / parts - r0) * (uint32_t)fnx;
+                        fy += 2 * (int)r0;
+                    }
                 }
-                walk_wide<kMS>(P, t, pay, large, quads, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY, keys, sp);
+                walk_wide<kMS>(P, t, pay, large, quads, fx, fy, fnx, tminX, tminY, tmaxX, tmaxY, keys, sp,
+                               (int)(4 * part / parts), (int)(4 * (part + 1) / parts));
             }
             if (until >= segEnd) {
                 if (nWide) __syncthreads();
