@@ -96,14 +96,16 @@ enum edxr_state_key {
     /* 1 = record HIP events around each pipeline stage of every frame. */
     EDXR_STATE_PROFILE = 3,
     /* 1 = capture each frame's launches in a HIP graph and replay it while the
-     * launch layout (sizes, capacities, tuning) repeats; default 0. */
+     * launch layout (sizes, capacities, tuning) repeats; default 0.  Frames on
+     * the direct path (below) are launched eagerly whatever this state is. */
     EDXR_STATE_GRAPH = 4,
     /* Triangles per binning chunk (0 = automatic: 1024, with at most 2,048
      * chunks per job of more than 4,096 tiles).  This setting and the next one
      * steer the general path only: small single-sample frames and batches (up
      * to 1,048,576 triangle slots, 416 per tile and 32,768 tiles, no bin chunks
-     * set) take a direct path, which lists references per tile without chunks
-     * or segments, unless a tile is too deep for it. */
+     * set for a single frame) take a direct path, which lists references per
+     * tile without chunks or segments, unless a tile is too deep for it.  Its
+     * lists take up to 16 KB of device memory per tile, kept by the context. */
     EDXR_STATE_TRIS_PER_CHUNK = 5,
     /* Raster work items per compute unit that the tile-segment size aims for
      * (0 = automatic, 8); the raster grid itself is always as many
@@ -134,7 +136,9 @@ enum edxr_state_key {
     EDXR_STATE_DEBUG_CAPACITY = 11
 };
 
-/* Pipeline stages timed when EDXR_STATE_PROFILE is on. */
+/* Pipeline stages timed when EDXR_STATE_PROFILE is on.  Frames on the direct
+ * path (EDXR_STATE_TRIS_PER_CHUNK) bin in their setup stage: the three binning
+ * stages take no time there. */
 enum edxr_stage {
     EDXR_STAGE_SETUP = 0,       /* vertex transform, outcodes, setup, clipping */
     EDXR_STAGE_BIN_COUNT = 1,
@@ -186,7 +190,8 @@ typedef struct edxr_stats {
     uint64_t refs;               /* tile references (N_ref) */
     uint64_t clip_vertices;      /* vertices created by clipping */
     uint32_t retries;            /* re-runs after a capacity overflow */
-    uint32_t bin_chunks;
+    uint32_t bin_chunks;         /* chunks of the general path's binning (also
+                                  * where the frame took the direct path) */
 } edxr_stats;
 
 /* One independent render job of a batch: a mesh, a camera, a light, a pixel
