@@ -117,6 +117,9 @@ class _RenderViews(torch.autograd.Function):
         ctx.njobs = len(views)
         ctx.V = V
         ctx.light_device = light.device
+        # The context's last render holds the addresses of these, which may be
+        # temporaries or contiguous copies: edxr_backward reads the mesh again.
+        ctx.mesh = (idx, planes)
         ctx.save_for_backward(px)
         return out
 
