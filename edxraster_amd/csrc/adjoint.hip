@@ -353,7 +353,7 @@ __global__ void k_adjoint_zero(double* acc, uint64_t nacc, double* vacc, uint64_
 // Adding every pixel's 27 values to the table with LDS atomics instead, where
 // the lanes of a triangle meet on the same addresses and look up its vertices
 // each, took 968 us for 64 views at 512 x 512 (3.8M covered pixels); this takes
-// 359 us, bound by the latency of its double-precision chains at three waves
+// 353 us, bound by the latency of its double-precision chains at three waves
 // per SIMD (168 VGPRs; about 1,200 vector instructions per 64 pixels).  Half
 // a tile per workgroup takes 388 us, a quarter 468 us, two waves per SIMD
 // without spills 425 us.

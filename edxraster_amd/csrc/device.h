@@ -779,7 +779,7 @@ struct TexLevel {
 // wrap per coordinate.  With a remainder per coordinate of every texel and the
 // levels found anew for every anisotropic tap, k_tile took 121 us for 8:1 at
 // 1080p (1.2M covered pixels, 64 texels each) and k_shade_tex 60 us for
-// trilinear at 1440p; so 90 and 56 us, now mostly the gathers' address rate.
+// trilinear at 1440p; so 84 and 51 us, now mostly the gathers' address rate.
 __device__ __forceinline__ float3 tex_bilinear(const FrameParams& P, const TexLevel& L, float u, float v) {
     const float x = u * (float)L.w - 0.5f, y = v * (float)L.h - 0.5f;
     const float x0 = floorf(x), y0 = floorf(y);
@@ -1293,9 +1293,9 @@ __device__ __forceinline__ void raster_item(const BatchParams& Q, const FramePar
             // last slice walked most of them, as heavy references end a tile's
             // list: 12 quad-walked and 10 tile-level ones made an item of 39 us
             // beside 12 on average, and the 2.1M sphere grid at 1080p took 45 us,
-            // 127 with 4 samples; so 36 and 86.  With a quadrant or 64 quads of each
-            // reference per wave its preparation by four waves cost more than the
-            // finer split gave: 40 and 86.)
+            // 127 with 4 samples; so 36 and 86 (34 and 78 with later steps).  With a
+            // quadrant or 64 quads of each reference per wave its preparation by four
+            // waves cost more than the finer split gave: 40 and 86.)
             const uint32_t nWide = __builtin_amdgcn_readfirstlane(min(wide->n, wide->limit));
             // With more samples and fewer references than waves, two or four waves
             // share each, by quadrants or by rows of quads: large triangles' tiles
